@@ -259,6 +259,7 @@ static int upload(htr_mix *m)
    if (rc) return rc;
    if (!m->host.constprop) build_species_reactions(m->host);
    for (int i = 0; i < m->host.nSpec; i++) derive_species(m->host.sp[i]);
+   if (!m->host.constprop) derive_transport(m->host);
    if (!m->dev && hipMalloc(&m->dev, sizeof(DMix)) != hipSuccess)
       return set_error(HTR_E_DEVICE, "mixture allocation failed");
    if (hipMemcpy(m->dev, &m->host, sizeof(DMix), hipMemcpyHostToDevice) != hipSuccess)

@@ -80,9 +80,9 @@ struct Diffusion {
       double heatFlux = interp2(t, P.lam, Q.lam)*m_s*(P.T - Q.T);
       double ViCorr = 0.0;
       double hs[NS];
+      MX::SpeciesEnthalpies(m, hs, T_s);
 #pragma unroll
       for (int i = 0; i < NS; i++) {
-         hs[i] = MX::SpeciesEnthalpy(m, i, T_s);
          const double YiVi = interp2(t, P.Di[i], Q.Di[i])*m_s*(P.X[i] - Q.X[i])*MX::SpeciesW(m, i)*iMixW_s;
          Flux[i] = -rho_s*YiVi;
          heatFlux += rho_s*YiVi*hs[i];

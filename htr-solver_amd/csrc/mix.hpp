@@ -20,6 +20,7 @@ constexpr int MAX_PD   = 4;
 constexpr int MAX_TB   = 8;
 
 constexpr double PI    = 3.1415926535898;
+constexpr double PI15  = 5.5683279968317265;     // PI^1.5
 constexpr double RGAS  = 8.3144598;
 constexpr double NA    = 6.02214086e23;
 constexpr double KB    = 1.38064852e-23;
@@ -41,6 +42,8 @@ struct DSpec {
    // [9] c4/3, [10] c5/6, [11] c6/5
    double cp[3][12];
    double rOvW;                // R/W, formed once at upload
+   double iW;                  // 1/W (correctly rounded, for quot())
+   double tHi, tLo;            // range switches: T > tHi takes cp[0] (infinite with two ranges), T > tLo cp[1]
    double sigma, kbOveps, mu, alpha, Z298;
 };
 
@@ -58,6 +61,10 @@ struct DReac {
 
 constexpr int MAX_SPR  = MAX_REAC*(MAX_ED + MAX_PD);
 
+// temperature-independent transport factors of a species and of a pair (i, j)
+struct DTran { double mu, fV, zrot, isk; };
+struct DPair { double w4, iw8, kT, iD; };
+
 struct DMix {
    int    constprop, nSpec, nReac, viscModel;
    double R, gamma, Prandtl;
@@ -67,6 +74,8 @@ struct DMix {
    double XiRef[MAX_SP];
    DSpec  sp[MAX_SP];
    DReac  rc[MAX_REAC];
+   DTran  tr[MAX_SP];
+   DPair  pr[MAX_SP][MAX_SP];
    // Species-major image of the stoichiometry, for the lane-per-species
    // accumulation of the production rates: the entries of species s are
    // [spr_ptr[s], spr_ptr[s+1]), in the order the reaction loop of
@@ -78,6 +87,25 @@ struct DMix {
 };
 
 #define HD __host__ __device__ inline
+
+// x/b given rb, the correctly rounded 1/b: the quotient of the product is
+// corrected twice by its exact residual, which makes it the correctly rounded
+// one (Markstein's theorem: the first correction brings it within one ulp, the
+// second rounds it correctly), and div_fixup restores the special values.
+// 6 FP64 operations against the 11 of a division; worth it wherever a divisor
+// is a constant of the mixture or serves several numerators.
+HD double quot(double x, double b, double rb)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+   double q = x*rb;
+   q = fma(fma(-b, q, x), rb, q);
+   q = fma(fma(-b, q, x), rb, q);
+   return __builtin_amdgcn_div_fixup(q, b, x);
+#else
+   (void)rb;
+   return x/b;
+#endif
+}
 
 // One thread's column of a shared species-major array: element i at
 // p[i*stride] (stride = threads of the block, so a wave's lanes touch
@@ -107,8 +135,46 @@ HD double conc_pow(double c, float nu)
 // ---------------------------------------------------------------- species --
 HD const double *cp_range(const DSpec &s, double T)
 {
-   if (s.nPoly == 3 && T > (double)s.TSwitch2) return s.cp[0];
-   return (T > (double)s.TSwitch1) ? s.cp[1] : s.cp[2];
+   return s.cp[T > s.tHi ? 0 : T > s.tLo ? 1 : 2];
+}
+
+// f(i, species i, its coefficients at T) for every species.  The range of a
+// polynomial is a lane's own, so its nine coefficients would be nine gathers
+// per species and evaluation, and the kernels that evaluate the polynomials
+// several times (temperature Newton, Roe state, face enthalpies) were bound by
+// them; nearly every wave has all its lanes in one range, and then the
+// coefficients come through scalar loads and enter as scalar operands.  A wave
+// that straddles a switch (and a mixture too large to hold its species'
+// ranges) gathers.  256^3 air: Roe pass 0.79 -> 0.71 ms per direction (233 ->
+// 147 VGPRs), diffusion species x 1.05 -> 0.86 ms.  The chemistry source
+// evaluates them once per cell and keeps the gathers (0.78 ms; 0.87 ms this
+// way, for a wave less per SIMD).
+template<int NS, class M, class F>
+HD void species_loop(const M &m, double T, F f)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+   if constexpr (NS <= 8) {
+      const uint64_t all = __ballot(1);
+      int r[NS];
+      bool one = true;
+#pragma unroll
+      for (int i = 0; i < NS; i++) {
+         const uint64_t hi = __ballot(T > m.sp[i].tHi), lo = __ballot(T > m.sp[i].tLo);
+         one = one && (hi == 0 || hi == all) && (lo == 0 || lo == all);
+         r[i] = hi ? 0 : lo ? 1 : 2;
+      }
+      if (one) {
+#pragma unroll
+         for (int i = 0; i < NS; i++) {
+            f(i, m.sp[i], m.sp[i].cp[r[i]]);
+            __builtin_amdgcn_sched_barrier(0);   // one species' scalars at a time
+         }
+         return;
+      }
+   }
+#endif
+#pragma unroll
+   for (int i = 0; i < NS; i++) f(i, m.sp[i], cp_range(m.sp[i], T));
 }
 
 // the quotients of DSpec formed at upload
@@ -120,106 +186,84 @@ inline void derive_species(DSpec &s)
       s.cp[r][11] = s.cp[r][6]/5;
    }
    s.rOvW = RGAS/s.W;
+   s.iW = 1.0/s.W;
+   s.tHi = (s.nPoly == 3) ? (double)s.TSwitch2 : HUGE_VAL;
+   s.tLo = (double)s.TSwitch1;
 }
 
-HD double sp_cp(const DSpec &s, double T)
+// polynomials on the coefficients c of a range (Species.inl:35-160)
+HD double poly_cp(const DSpec &s, const double *c, double T, double Tinv)
 {
-   const double rOvW = s.rOvW;
-   const double Tinv = 1.0/T;
-   const double *c = cp_range(s, T);
    const double poly = c[3] + T*(c[4] + T*(c[5] + T*c[6]));
-   return rOvW*(c[0]*Tinv*Tinv + c[1]*Tinv + c[2] + T*poly);
+   return s.rOvW*(c[0]*Tinv*Tinv + c[1]*Tinv + c[2] + T*poly);
 }
 
-HD double sp_free_enthalpy(const DSpec &s, double T)
+HD double poly_free_enthalpy(const double *c, double T, double Tinv, double logT)
 {
-   const double Tinv = 1.0/T;
-   const double logT = log(T);
-   const double *c = cp_range(s, T);
    const double G = -0.5*c[0]*Tinv*Tinv + c[1]*Tinv*(1.0 + logT) + c[2]*(1.0 - logT) + c[7]*Tinv - c[8];
    return G - 0.5*T*(c[3] + T*(c[9] + T*(c[10] + 0.1*T*c[6])));
 }
 
-HD double sp_enthalpy(const DSpec &s, double T)
+HD double poly_enthalpy(const DSpec &s, const double *c, double T, double Tinv, double logT)
 {
-   const double rOvW = s.rOvW;
-   const double Tinv = 1.0/T;
-   const double *c = cp_range(s, T);
-   const double E = -c[0]*Tinv + c[1]*log(T) + c[7] + T*(c[2] + T*(c[3]*0.50 + T*(c[9] + T*(c[5]*0.25 + c[11]*T))));
-   return E*rOvW;
+   const double E = -c[0]*Tinv + c[1]*logT + c[7] + T*(c[2] + T*(c[3]*0.50 + T*(c[9] + T*(c[5]*0.25 + c[11]*T))));
+   return E*s.rOvW;
 }
 
-HD double omega_mu(double T)
-{
-   const double num = 3.3530622607 + T*(2.53272006 + T*(2.9024238575 + T*0.11186138893));
-   const double den = 0.8662326188 + T*(1.3913958626 + T*(3.158490576 + T*(0.18973411754 + T*0.00018682962894)));
-   return num/den;
-}
+HD double sp_cp(const DSpec &s, double T) { return poly_cp(s, cp_range(s, T), T, 1.0/T); }
+HD double sp_free_enthalpy(const DSpec &s, double T) { return poly_free_enthalpy(cp_range(s, T), T, 1.0/T, log(T)); }
+HD double sp_enthalpy(const DSpec &s, double T) { return poly_enthalpy(s, cp_range(s, T), T, 1.0/T, log(T)); }
 
-HD double omega_D(double T)
-{
-   const double num = 6.8728271691 + T*(9.4122316321 + T*(7.7442359037 + T*0.23424661229));
-   const double den = 1.45337701568 + T*(5.2269794238 + T*(9.7108519575 + T*(0.46539437353 + T*0.00041908394781)));
-   return num/den;
-}
+// Collision integrals (Species.inl:163-190) as numerator and denominator: the
+// transport properties divide by them, so a quotient of theirs is formed once
+// with the other factors
+HD double omega_mu_num(double T) { return 3.3530622607 + T*(2.53272006 + T*(2.9024238575 + T*0.11186138893)); }
+HD double omega_mu_den(double T)
+{ return 0.8662326188 + T*(1.3913958626 + T*(3.158490576 + T*(0.18973411754 + T*0.00018682962894))); }
+HD double omega_D_num(double T) { return 6.8728271691 + T*(9.4122316321 + T*(7.7442359037 + T*0.23424661229)); }
+HD double omega_D_den(double T)
+{ return 1.45337701568 + T*(5.2269794238 + T*(9.7108519575 + T*(0.46539437353 + T*0.00041908394781))); }
 
-HD double sp_mu(const DSpec &s, double T)
+// Rotational relaxation factor (Species.inl:290-295) of T* = kbOveps T
+inline double sp_fzrot(double kbOveps, double T)
 {
-   const double num = 5*sqrt(PI*s.W/NA*KB*T);
-   const double den = 16*PI*pow(s.sigma, 2.0)*omega_mu(T*s.kbOveps);
-   return num/den;
-}
-
-HD double sp_dif(const DSpec &a, const DSpec &b, double P, double T)
-{
-   double xi = 1.0;
-   if ((a.mu*b.mu == 0.0) && (a.mu + b.mu != 0.0)) {
-      double mup, alp, epr;
-      if (a.mu != 0.0) {
-         mup = a.mu/sqrt(4*PI*EPS0*KB*pow(a.sigma, 3.0)/a.kbOveps);
-         alp = b.alpha/pow(b.sigma, 3.0);
-         epr = sqrt(b.kbOveps/a.kbOveps);
-      } else {
-         mup = b.mu/sqrt(4*PI*EPS0*KB*pow(b.sigma, 3.0)/b.kbOveps);
-         alp = a.alpha/pow(a.sigma, 3.0);
-         epr = sqrt(a.kbOveps/b.kbOveps);
-      }
-      xi = 1 + 0.25*mup*alp*epr;
-   }
-   const double sigmaij = 0.5*(a.sigma + b.sigma)*pow(xi, -1./6);
-   const double kboEpsij = sqrt(a.kbOveps*b.kbOveps)/(xi*xi);
-   const double omega11 = omega_D(T*kboEpsij);
-   const double invWij = (a.W + b.W)/(a.W*b.W);
-   const double num = 3*sqrt(2*PI*pow(KB, 3.0)*pow(T, 3.0)*NA*invWij);
-   const double den = 16*PI*P*sigmaij*sigmaij*omega11;
-   return num/den;
-}
-
-HD double sp_fzrot(const DSpec &s, double T)
-{
-   const double tmp = 1.0/(s.kbOveps*T);
+   const double tmp = 1.0/(kbOveps*T);
    return 1 + 0.5*pow(PI, 1.5)*sqrt(tmp) + (2 + 0.25*PI*PI)*tmp + pow(PI, 1.5)*pow(tmp, 1.5);
 }
 
-HD double sp_lam(const DSpec &s, double T)
+// The temperature-independent factors of the species' and pairs' transport
+// properties, formed once when a mixture is uploaded
+inline void derive_transport(DMix &m)
 {
-   if (s.geom == GEOM_ATOM) {
-      const double mu = sp_mu(s, T);
-      return 15.0/4*mu*RGAS/s.W;
+   for (int i = 0; i < m.nSpec; i++) {
+      const DSpec &s = m.sp[i];
+      DTran &t = m.tr[i];
+      // Species.inl:193-199: mu = 5 sqrt(PI W/NA KB T)/(16 PI sigma^2 omega)
+      t.mu = 5*sqrt(PI*s.W/NA*KB)/(16*PI*pow(s.sigma, 2.0));
+      // Species.inl:310-357: the self-diffusion factor over mu
+      t.fV = 3*sqrt(PI*KB*s.W/NA)/(8*PI*pow(s.sigma, 2.0))/t.mu;
+      t.zrot = s.Z298*sp_fzrot(s.kbOveps, 298);
+      t.isk = 1.0/sqrt(s.kbOveps);
+      for (int j = 0; j < m.nSpec; j++) {
+         const DSpec &o = m.sp[j];
+         DPair &p = m.pr[i][j];
+         // Wilke's rule: Phi = (1 + sqrt(mu_i/mu_j) (W_j/W_i)^(1/4))^2/sqrt(8 (1 + W_i/W_j))
+         p.w4 = pow(o.W/s.W, 0.25);
+         p.iw8 = 1.0/sqrt(8*(1 + s.W/o.W));
+         // Species.inl:225-288: binary diffusivity D = 3 sqrt(2 PI KB^3 T^3 NA/W_ij)/(16 PI P sigma_ij^2 omega)
+         double xi = 1.0;
+         if ((s.mu*o.mu == 0.0) && (s.mu + o.mu != 0.0)) {
+            const DSpec &a = (s.mu != 0.0) ? s : o, &b = (s.mu != 0.0) ? o : s;   // polar, non-polar
+            const double mup = a.mu/sqrt(4*PI*EPS0*KB*pow(a.sigma, 3.0)/a.kbOveps);
+            const double alp = b.alpha/pow(b.sigma, 3.0);
+            xi = 1 + 0.25*mup*alp*sqrt(b.kbOveps/a.kbOveps);
+         }
+         const double sigmaij = 0.5*(s.sigma + o.sigma)*pow(xi, -1./6);
+         const double invWij = (s.W + o.W)/(s.W*o.W);
+         p.kT = sqrt(s.kbOveps*o.kbOveps)/(xi*xi);
+         p.iD = 16*PI*sigmaij*sigmaij/(3*sqrt(2*PI*pow(KB, 3.0)*NA*invWij));
+      }
    }
-   const double CvROvR = (s.geom == GEOM_LINEAR) ? 1.0 : 1.5;
-   const double CvT = 1.5*RGAS;
-   const double CvR = CvROvR*RGAS;
-   const double CvV = (s.geom == GEOM_LINEAR) ? sp_cp(s, T)*s.W - 3.5*RGAS : sp_cp(s, T)*s.W - 4.0*RGAS;
-   const double Dkk = 3*sqrt(PI*KB*T*s.W/NA)/(8*PI*pow(s.sigma, 2.0)*omega_D(T*s.kbOveps));
-   const double mu = sp_mu(s, T);
-   const double fV = Dkk/mu;
-   const double Zrot = s.Z298*sp_fzrot(s, 298)/sp_fzrot(s, T);
-   const double A = 2.5 - fV;
-   const double B = Zrot + 2/PI*(5./3*CvROvR + fV);
-   const double fT = 2.5*(1. - 2*CvR*A/(PI*CvT*B));
-   const double fR = fV*(1. + 2*A/(PI*B));
-   return mu/s.W*(fT*CvT + fR*CvR + fV*CvV);
 }
 
 // ---------------------------------------------------------------- mixture --
@@ -234,7 +278,7 @@ struct Mix {
    {
       if (CP) return RGAS/m.R;
       double W = 0.0;
-      for (int i = 0; i < NS; i++) W += Y[i]/m.sp[i].W;
+      for (int i = 0; i < NS; i++) W += quot(Y[i], m.sp[i].W, m.sp[i].iW);
       return 1.0/W;
    }
    HD static double MolarWeightFromX(const DMix &m, const double *X)
@@ -247,12 +291,13 @@ struct Mix {
    HD static void MolarFractions(const DMix &m, double *X, double MixW, const double *Y)
    {
       if (CP) { X[0] = Y[0]; return; }
-      for (int i = 0; i < NS; i++) X[i] = Y[i]*MixW/m.sp[i].W;
+      for (int i = 0; i < NS; i++) X[i] = quot(Y[i]*MixW, m.sp[i].W, m.sp[i].iW);
    }
    HD static void MassFractions(const DMix &m, double *Y, double MixW, const double *X)
    {
       if (CP) { Y[0] = X[0]; return; }
-      for (int i = 0; i < NS; i++) Y[i] = X[i]*m.sp[i].W/MixW;
+      const double iMixW = 1.0/MixW;
+      for (int i = 0; i < NS; i++) Y[i] = quot(X[i]*m.sp[i].W, MixW, iMixW);
    }
    HD static double SpeciesW(const DMix &m, int i) { return CP ? RGAS/m.R : m.sp[i].W; }
    HD static double Rho(const DMix &m, double P, double T, double MixW)
@@ -264,8 +309,9 @@ struct Mix {
    {
       if (CP) return m.gamma/(m.gamma - 1)*m.R;
       const double T = Tn*m.TRef;
+      const double Tinv = 1.0/T;
       double cp = 0.0;
-      for (int i = 0; i < NS; i++) cp += Y[i]*sp_cp(m.sp[i], T);
+      species_loop<NS>(m, T, [&](int i, const DSpec &s, const double *c) { cp += Y[i]*poly_cp(s, c, T, Tinv); });
       return cp*m.iCpRef;
    }
    HD static double SpeciesEnthalpy(const DMix &m, int i, double T)
@@ -273,12 +319,22 @@ struct Mix {
       if (CP) return m.gamma/(m.gamma - 1)*m.R*T;
       return sp_enthalpy(m.sp[i], T*m.TRef)*m.ieRef;
    }
+   // all species at once (the face enthalpies of the diffusion)
+   HD static void SpeciesEnthalpies(const DMix &m, double *h, double Tn)
+   {
+      if (CP) { h[0] = m.gamma/(m.gamma - 1)*m.R*Tn; return; }
+      const double T = Tn*m.TRef, Tinv = 1.0/T, logT = log(T);
+      species_loop<NS>(m, T, [&](int i, const DSpec &s, const double *c) { h[i] = poly_enthalpy(s, c, T, Tinv, logT)*m.ieRef; });
+   }
    HD static double InternalEnergy(const DMix &m, double Tn, const double *Y)
    {
       if (CP) return Tn*m.R/(m.gamma - 1.0);
       const double T = Tn*m.TRef;
+      const double Tinv = 1.0/T, logT = log(T), RT = RGAS*T;
       double e = 0.0;
-      for (int i = 0; i < NS; i++) e += Y[i]*(sp_enthalpy(m.sp[i], T) - RGAS*T/m.sp[i].W);
+      species_loop<NS>(m, T, [&](int i, const DSpec &s, const double *c) {
+         e += Y[i]*(poly_enthalpy(s, c, T, Tinv, logT) - quot(RT, s.W, s.iW));
+      });
       return e*m.ieRef;
    }
    // MultiComponent.inl:187-210; iters (optional) receives the Newton count
@@ -290,8 +346,11 @@ struct Mix {
       while (j < 1000) {
          const double f = e0 - InternalEnergy(m, T, Y);
          if (fabs(f/dfdT) < 1e-8) break;
+         const double Td = T*m.TRef, Tinv = 1.0/Td;
          dfdT = 0.0;
-         for (int i = 0; i < NS; i++) dfdT += Y[i]*(sp_cp(m.sp[i], T*m.TRef) - m.sp[i].rOvW)*m.iCpRef;
+         species_loop<NS>(m, Td, [&](int i, const DSpec &s, const double *c) {
+            dfdT += Y[i]*(poly_cp(s, c, Td, Tinv) - s.rOvW)*m.iCpRef;
+         });
          T += f/dfdT;
          j++;
       }
@@ -314,38 +373,98 @@ struct Mix {
       if (m.viscModel == VISC_POWERLAW) return m.plVRef*pow((T/m.plTRef), 0.7);
       return (m.suVRef*pow((T/m.suTRef), 1.5))*((m.suTRef + m.suSRef)/(T + m.suSRef));
    }
-   HD static double Viscosity(const DMix &m, double Tn, const double *X)
-   {
-      if (CP) return ConstVisc(m, Tn);
-      const double T = Tn*m.TRef;
-      double muk[NS];
-      for (int i = 0; i < NS; i++) muk[i] = sp_mu(m.sp[i], T);
-      double mu = 0.0;
-      for (int i = 0; i < NS; i++) {
-         double den = 0.0;
-         for (int j = 0; j < NS; j++) {
-            double Phi = 1 + sqrt(muk[i]/muk[j])*pow(m.sp[j].W/m.sp[i].W, 0.25);
-            Phi *= Phi/sqrt(8*(1 + m.sp[i].W/m.sp[j].W));
-            den += X[j]*Phi;
-         }
-         mu += X[i]*muk[i]/den;
-      }
-      return mu*m.imuRef;
-   }
-   HD static double HeatConductivity(const DMix &m, double Tn, const double *X)
+   // Viscosity (Wilke), heat conductivity, diffusivities and the speed of
+   // sound of one cell (MultiComponent.inl:215-330, Species.inl:193-357).  Formed
+   // together they share sqrt(T), the species viscosities (which the
+   // conductivities need too), the heat capacities (which the speed of sound
+   // needs too) and the factors of derive_transport: one quotient per pair and
+   // collision integral, no pow, and one square root per species.  Bound by
+   // FP64 issue when each property formed its own factors with pow and sqrt
+   // (4200 FP64 instructions per cell); the fused stage update of 160^3 air
+   // went from 2.14 to 0.52 ms, 3.8 TB/s of its 480 B per cell, with Newton
+   // and properties together.
+   HD static void Transport(const DMix &m, double Pn, double Tn, double MixW, const double *X, const double *Y,
+                            double &muOut, double &lamOut, double *Di, double &SoS)
    {
       if (CP) {
          const double cp = m.gamma/(m.gamma - 1)*m.R;
-         return cp/m.Prandtl*ConstVisc(m, Tn);
+         const double visc = ConstVisc(m, Tn);
+         muOut = visc;
+         lamOut = cp/m.Prandtl*visc;
+         Di[0] = 0.0;
+         SoS = sqrt(m.gamma*m.R*Tn);
+         return;
       }
-      const double T = Tn*m.TRef;
-      double a = 0.0, b = 0.0;
+      const double T = Tn*m.TRef, P = Pn*m.PRef;
+      const double sT = sqrt(T), Tinv = 1.0/T, isT = sT*Tinv;
+      double sk[NS], isk[NS], cpm = 0.0, la = 0.0, lb = 0.0;
+      species_loop<NS>(m, T, [&](int i, const DSpec &s, const double *c) {
+         const DTran &tr = m.tr[i];
+         const double Ts = T*s.kbOveps;
+         const double on = omega_mu_num(Ts), od = omega_mu_den(Ts);
+         const double mu = tr.mu*sT*od/on;
+         sk[i] = sqrt(mu);
+         isk[i] = 1.0/sk[i];
+         const double cp = poly_cp(s, c, T, Tinv);
+         cpm += Y[i]*cp;
+         double lam;
+         if (s.geom == GEOM_ATOM) {
+            lam = 15.0/4*mu*s.rOvW;
+         } else {
+            const bool lin = (s.geom == GEOM_LINEAR);
+            const double CvROvR = lin ? 1.0 : 1.5;
+            const double CvT = 1.5*RGAS, CvR = CvROvR*RGAS;
+            const double CvV = cp*s.W - (lin ? 3.5 : 4.0)*RGAS;
+            const double fV = tr.fV*omega_D_den(Ts)*on/(omega_D_num(Ts)*od);
+            const double r1 = tr.isk*isT, r2 = r1*r1;      // sqrt(1/T*), 1/T*
+            const double fz = 1 + 0.5*PI15*r1 + (2 + 0.25*PI*PI)*r2 + PI15*(r2*r1);
+            const double A = 2.5 - fV;
+            // A/B with B = zrot/fz + 2/PI (5/3 CvR/R + fV)
+            const double AB = A*fz/(tr.zrot + fz*(2/PI*(5./3*CvROvR + fV)));
+            const double fT = 2.5*(1. - 2*CvR/(PI*CvT)*AB);
+            const double fR = fV*(1. + 2/PI*AB);
+            lam = mu*s.iW*(fT*CvT + fR*CvR + fV*CvV);
+         }
+         la += X[i]*lam;
+         lb += X[i]/lam;
+      });
+      lamOut = 0.5*(la + 1.0/lb)*m.ilamRef;
+      double mu = 0.0;
+#pragma unroll
       for (int i = 0; i < NS; i++) {
-         const double lami = sp_lam(m.sp[i], T);
-         a += X[i]*lami;
-         b += X[i]/lami;
+         double den = 0.0;
+#pragma unroll
+         for (int j = 0; j < NS; j++) {
+            if (j == i) { den += X[j]; continue; }         // Phi = 1
+            const double phi = 1 + sk[i]*isk[j]*m.pr[i][j].w4;
+            den += X[j]*(phi*phi*m.pr[i][j].iw8);
+         }
+         mu += X[i]*(sk[i]*sk[i])/den;
       }
-      return 0.5*(a + 1.0/b)*m.ilamRef;
+      muOut = mu*m.imuRef;
+#pragma unroll
+      for (int i = 0; i < NS; i++) Di[i] = 0.0;
+      const double PT = P*(Tinv*isT);                      // P/T^(3/2)
+#pragma unroll
+      for (int i = 0; i < NS; i++)
+#pragma unroll
+         for (int j = 0; j < i; j++) {
+            const DPair &p = m.pr[i][j];
+            const double Ts = T*p.kT;
+            const double invDij = p.iD*PT*omega_D_num(Ts)/omega_D_den(Ts);
+            Di[i] += X[j]*invDij;
+            Di[j] += X[i]*invDij;
+         }
+#pragma unroll
+      for (int i = 0; i < NS; i++) {
+         double num = 0.0;
+#pragma unroll
+         for (int j = 0; j < NS; j++)
+            if (j != i) num += X[j]*m.sp[j].W;
+         Di[i] = num/(MixW*Di[i])*m.iDiRef;
+      }
+      const double cp = cpm*m.iCpRef, Wr = MixW*m.iMixWRef;
+      SoS = SpeedOfSound(m, Tn, cp/(cp - 1.0/Wr), MixW);
    }
    HD static double Gamma(const DMix &m, double T, double MixW, const double *Y)
    {
@@ -359,36 +478,18 @@ struct Mix {
       if (CP) return sqrt(gamma*m.R*T);
       return sqrt(gamma*T/(MixW*m.iMixWRef));
    }
-   HD static void Diffusivity(const DMix &m, double *Di, double Pn, double Tn, double MixW, const double *X)
-   {
-      if (CP) { Di[0] = 0.0; return; }
-      const double T = Tn*m.TRef;
-      const double P = Pn*m.PRef;
-      for (int i = 0; i < NS; i++) Di[i] = 0.0;
-      for (int i = 0; i < NS; i++)
-         for (int j = 0; j < i; j++) {
-            const double invDij = 1.0/sp_dif(m.sp[i], m.sp[j], P, T);
-            Di[i] += X[j]*invDij;
-            Di[j] += X[i]*invDij;
-         }
-      for (int i = 0; i < NS; i++) {
-         double num = 0.0;
-         for (int j = 0; j < NS; j++)
-            if (j != i) num += X[j]*m.sp[j].W;
-         Di[i] = num/(MixW*Di[i])*m.iDiRef;
-      }
-   }
    HD static double dpde(double rho, double gamma) { return rho*(gamma - 1); }
    HD static void dpdrhoi(const DMix &m, double *d, double gamma, double Tn, const double *Y)
    {
       if (CP) { d[0] = m.R*Tn; return; }
       const double T = Tn*m.TRef;
+      const double Tinv = 1.0/T, logT = log(T), RT = RGAS*T;
       double e = 0.0;
-      for (int i = 0; i < NS; i++) {
-         d[i] = sp_enthalpy(m.sp[i], T) - RGAS*T/m.sp[i].W;
+      species_loop<NS>(m, T, [&](int i, const DSpec &s, const double *c) {
+         d[i] = poly_enthalpy(s, c, T, Tinv, logT) - quot(RT, s.W, s.iW);
          e += Y[i]*d[i];
-      }
-      for (int i = 0; i < NS; i++) d[i] = (RGAS*T/m.sp[i].W + (gamma - 1)*(e - d[i]))*m.ieRef;
+      });
+      for (int i = 0; i < NS; i++) d[i] = (quot(RT, m.sp[i].W, m.sp[i].iW) + (gamma - 1)*(e - d[i]))*m.ieRef;
    }
 
    // Reaction.inl:34-42: Kf = A T^n exp(-EovR/T), formed as
@@ -410,12 +511,12 @@ struct Mix {
       const double T = Tn*m.TRef;
       const double P = Pn*m.PRef;
       const double rho = rhon*m.rhoRef;
+      const double logT = log(T), Tinv = 1.0/T;
       for (int i = 0; i < NS; i++) {
          w[i] = 0.0;
          C[i] = Y[i]*rho/m.sp[i].W;
-         G[i] = sp_free_enthalpy(m.sp[i], T);
+         G[i] = poly_free_enthalpy(cp_range(m.sp[i], T), T, Tinv, logT);
       }
-      const double logT = log(T);
       const double logRP = log(RGAS/P);
       for (int k = 0; k < m.nReac; k++) {
          const DReac &r = m.rc[k];

@@ -31,17 +31,16 @@ __device__ __forceinline__ void properties_to(const htr_fields &f, const DMix &m
                                               const double *X)
 {
    constexpr int NS = MX::NS;
-   double Y[NS], D[NS];
+   double Y[NS], D[NS], mu, lam, c;
    const double MixW = MX::MolarWeightFromX(m, X);
-   at<double>(f.rho, p) = MX::Rho(m, P, T, MixW);
-   at<double>(f.mu, p) = MX::Viscosity(m, T, X);
-   at<double>(f.lam, p) = MX::HeatConductivity(m, T, X);
-   MX::Diffusivity(m, D, P, T, MixW, X);
    MX::MassFractions(m, Y, MixW, X);
+   MX::Transport(m, P, T, MixW, X, Y, mu, lam, D, c);
+   at<double>(f.rho, p) = MX::Rho(m, P, T, MixW);
+   at<double>(f.mu, p) = mu;
+   at<double>(f.lam, p) = lam;
 #pragma unroll
    for (int i = 0; i < NS; i++) { at<double>(f.Di, p, i) = D[i]; at<double>(f.MassFracs, p, i) = Y[i]; }
-   const double gamma = MX::Gamma(m, T, MixW, Y);
-   at<double>(f.SoS, p) = MX::SpeedOfSound(m, T, gamma, MixW);
+   at<double>(f.SoS, p) = c;
 }
 
 template<class MX>
