@@ -888,43 +888,40 @@ euler_roe_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, 
    }
 }
 
-// Passes 2b + 2c in one kernel, pipelined: a block of four waves takes
-// chunks of 64 listed TENO faces.
-//   components  waves 0, 1, 2 form the components they own (wave 0 one of
-//               nine, waves 1 and 2 four each) of the 64 faces of chunk k
-//               from the stencil-point values in LDS (the component index is
-//               wave-uniform, so every branch on it is uniform): per point
-//               the species sums of the left-eigenvector products
-//               (rhs.inl:443-451), the split fluxes on row i, TENO+ and
-//               TENO-, -(F+ + F-)/2 and the stencil-selection bits into LDS
-//               (double-buffered by chunk parity);
-//   finish      wave 0, before its component of chunk k: back-projects
-//               chunk k - 1 (add_column, the reference's summation order),
-//               tests the limiter, writes the face fluxes and decision words
-//               and lists the faces that need the limiter blend;
-//   loader      wave 3, meanwhile: issues the gathers of chunk k + 1's
-//               stencil-point values (conserved vector, u_n, p: 6 (nEq + 2)
-//               doubles per face) into its registers;
-//   hand-over   after the component waves are done with chunk k, the loader
-//               writes chunk k + 1's values, face ids and node types into
-//               LDS.
-// The scattered gathers thus fly while the components of the previous chunk
-// are computed; only the LDS write of the hand-over is on the component
-// waves' path.  The Roe record of a face (euler_roe_kernel) is read by the
-// component waves where it is used, with coalesced loads (list order =
-// record order).  44 KB of LDS per block (air): three blocks, twelve waves
-// per CU.
+// Passes 2b + 2c in one kernel.  A block of four waves takes chunks of 64
+// listed TENO faces, a lane per face, in three steps between barriers:
+//   stage       the six stencil points, dealt to the waves: the point's
+//               values (conserved vector, u_n, p) are gathered and left in
+//               LDS with its four species sums of the left-eigenvector
+//               products (rhs.inl:443-451), formed once and not again for
+//               each of the nine components that use them;
+//   components  the nEq components, dealt to the waves (the component index
+//               is wave-uniform, so every branch on it is): split fluxes of
+//               the six points on row i, TENO+ and TENO-, -(F+ + F-)/2 and
+//               the stencil-selection bits into LDS;
+//   finish      the last wave, before it stages the next chunk:
+//               back-projection (add_column, the reference's summation
+//               order), limiter test, face fluxes, decision words, and the
+//               list of the faces that need the limiter blend.
+// The steps of a block do not overlap; the three blocks of a CU (52 KB of LDS
+// each) do, and no wave is kept for loading alone.  Bound by the latency of
+// the gathers: its waves wait 74 % of their cycles.  256^3 air, per y or z
+// sweep (3.36 M TENO faces): 2.17 ms, against 2.38 ms with the sums formed per
+// component and the gathers of a loading wave overlapped; 128^3 with 85 % TENO
+// faces 0.81 against 0.97 ms.
 constexpr int TENO_WAVES = 4;
 
 template<class MX>
 struct TenoStage {
    static constexpr int NS = MX::NS, NEQ = MX::NEQ;
-   static constexpr int NPV = NS + 6;                // per point: rhoY_0..NS-1, rhou 3, rhoE, u_n, p
+   // per point: rhoY_0..NS-1, rhou 3, rhoE, u_n, p, then the species sums of
+   // the conserved vector (weighted, plain) and of the flux
+   static constexpr int UN = NS + 4, PR = NS + 5, S1Q = NS + 6, SQQ = NS + 7, S1F = NS + 8, SQF = NS + 9;
+   static constexpr int NPV = NS + 10;
    double  pt[6*NPV][64];
-   double  fc[2][NEQ][64];
-   uint8_t bits[2][NEQ][64];
-   uint32_t fid[2][64];                             // face id and node type of the chunk's faces,
-   int32_t  ty[2][64];                              // by chunk parity (left by the loader)
+   double  fc[NEQ][64];
+   double  w[16][4];                                // StdWeights
+   uint8_t bits[NEQ][64];
 };
 
 template<class MX, int DIR, int SCHEME, bool LISTED>
@@ -936,11 +933,10 @@ euler_teno_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g,
 {
    using E_t = Euler<MX, DIR>;
    using St = TenoStage<MX>;
-   const double dt = dta.get();
    constexpr int NS = MX::NS, NEQ = MX::NEQ, NPV = St::NPV;
    constexpr int OP = (SCHEME == HTR_EULER_TENOA) ? 1 : (SCHEME == HTR_EULER_TENOLAD) ? 2 : 0;
    constexpr int iN = E_t::iN;
-   constexpr int LOADER = TENO_WAVES - 1;
+   constexpr int LAST = TENO_WAVES - 1;
    __shared__ St S;
    const uint32_t n = (uint32_t)(LISTED ? (int64_t)counter[1] : nfaces);
    const uint32_t nchunks = (n + 63u)/64u;
@@ -948,69 +944,37 @@ euler_teno_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g,
    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
    const int64_t cap = b.cap;
    E_t E{f, *mix, g, hv};
-   // chunks of this block: L + k gridDim.x, k = 0 .. K - 1, with L the
-   // XCD-aware logical block index (the chunks in flight on one XCD are
-   // neighbours in the list and share stencil cache lines)
+   // chunks of this block: L + k gridDim.x, with L the XCD-aware logical block
+   // index (the chunks in flight on one XCD are neighbours in the list and
+   // share stencil cache lines)
    const uint32_t L = xcd_block(blockIdx.x, gridDim.x);
-   const uint32_t K = (L < nchunks) ? (nchunks - 1u - L)/gridDim.x + 1u : 0u;
-   auto chunk = [&](uint32_t k) { return L + k*gridDim.x; };
+   if (L >= nchunks) return;                         // uniform over the block
+   const double dt = dta.get();
+   if (threadIdx.x < 64) S.w[lane >> 2][lane & 3] = c_stdw.w[lane >> 2][lane & 3];
 
-   // the face's cell and node type, from the ids and node types the loader
-   // left in LDS (buffer bb): no dependent global loads before the face's work
-   auto face_lds = [&](int bb, P3 &q, int &t) {
-      q = Faces<DIR>::cell(g, f, S.fid[bb][lane]);
-      t = S.ty[bb][lane];
-   };
-
-   // loader: the stencil-point values of the 64 faces of chunk c into pv,
-   // the face id and node type into fi, ti
-   auto gather = [&](uint32_t c, double *pv, uint32_t &fi, int &ti) {
+   // face id, left cell and node type of the lane's face of chunk c; past the
+   // list's end the first cell stands in (its values are not used)
+   uint32_t fid = 0;
+   P3 q;
+   int t = 0;
+   auto face = [&](uint32_t c) {
       const uint32_t w = c*64u + (uint32_t)lane;
-      const bool valid = w < n;
-      P3 P[6];
-      fi = 0;
-      ti = 0;
-      if (valid) {
-         P3 q;
-         int t;
-         fi = LISTED ? (uint32_t)list[w] : w;
-         q = Faces<DIR>::cell(g, f, fi);
+      fid = 0;
+      t = Std_node;
+      q = mkp(g, 0, 0, 0);
+      if (w < n) {
+         fid = LISTED ? (uint32_t)list[w] : w;
+         q = Faces<DIR>::cell(g, f, fid);
          t = ld<int>(f.nType[DIR], q);
-         ti = t;
-         E.points(P, q, t);
       }
-      if (!valid)
-#pragma unroll
-         for (int k = 0; k < 6; k++) P[k] = mkp(g, 0, 0, 0);      // a valid point; the values are not used
-      // one point at a time: the addresses of the next point's loads are
-      // formed after this point's loads are issued (hoisted, they would hold
-      // some 100 VGPRs next to the 6 (nEq + 2) values)
-#pragma unroll
-      for (int k = 0; k < 6; k++) {
-         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-         for (int v = 0; v < NPV; v++)
-            pv[k*NPV + v] = (v < NS + 4) ? ld<double>(f.Conserved, P[k], v)
-                          : (v == NS + 4) ? ld<double>(f.velocity, P[k], iN) : ld<double>(f.pressure, P[k]);
-      }
-   };
-   auto hand_over = [&](const double *pv, uint32_t fi, int ti, int bb) {
-#pragma unroll
-      for (int k = 0; k < 6*NPV; k++) S.pt[k][lane] = pv[k];
-      S.fid[bb][lane] = fi;
-      S.ty[bb][lane] = ti;
    };
 
-   // loader: back-projection, limiter test, face flux and decision word of
-   // the 64 faces of chunk c, whose components are in buffer bb
-   // (rhs.inl:708-721)
-   auto finish = [&](uint32_t c, int bb) {
+   // back-projection, limiter test, face flux and decision word of the lane's
+   // face of chunk c (rhs.inl:708-721)
+   auto finish = [&](uint32_t c) {
       const uint32_t w = c*64u + (uint32_t)lane;
       bool limit = false;
       if (w < n) {
-         P3 q;
-         int t;
-         face_lds(bb, q, t);
          typename E_t::Roe R;
          E_t::get_rec(b.rec, cap, w, R);
          const double dedp = 1.0/R.dpde;
@@ -1020,8 +984,8 @@ euler_teno_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g,
          uint32_t h = 0;
 #pragma unroll
          for (int i = 0; i < NEQ; i++) {
-            E_t::add_column(Flux, sumQsp, i, S.fc[bb][i][lane], R, ERoe, dedp);
-            const uint32_t bt = S.bits[bb][i][lane];
+            E_t::add_column(Flux, sumQsp, i, S.fc[i][lane], R, ERoe, dedp);
+            const uint32_t bt = S.bits[i][lane];
             h = fold_bits(fold_bits(h, bt & 15u), bt >> 4);
          }
          if (NS > 1) {
@@ -1035,7 +999,6 @@ euler_teno_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g,
                   limit = true;
             }
          }
-         const uint32_t fid = S.fid[bb][lane];
          store_face<NEQ>(F, nfaces, fid, Flux);
          if (dec.ptr) at<uint32_t>(dec, q) = h << 2;
       }
@@ -1049,117 +1012,88 @@ euler_teno_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g,
       }
    };
 
-   // component waves: the components of chunk c that the wave owns into
-   // buffer bb.  Owner of component i: the pattern 1, 2, 1, 2, 0, 2, 1, 2, 1
-   // (nine components: wave 0 one, waves 1 and 2 four each), since wave 0
-   // also back-projects the previous chunk (timed per role, an even three
-   // each made wave 0 the critical path of every chunk).
-   auto owner = [](int i) { const int r = i % 9; return (r == 4) ? 0 : (r & 1) ? 2 : 1; };
-   auto components = [&](uint32_t c, int bb) {
+   for (uint32_t c = L; c < nchunks; c += gridDim.x) {
+      if (wv == LAST && c != L) finish(c - gridDim.x);
+      face(c);
       const uint32_t w = c*64u + (uint32_t)lane;
-      const bool valid = w < n;
-      int tt = 0;
-      if (valid) tt = S.ty[bb][lane];
-      const bool all_std = __ballot(tt != Std_node) == 0ull;
-      if (!valid) return;
+      const uint32_t wr = w < n ? w : n - 1u;        // a record that exists
       typename E_t::Roe R;
-#pragma unroll
-      for (int j = 0; j < 3; j++) R.v[j] = b.rec[(int64_t)(NS + j)*cap + w];
-      R.a = b.rec[(int64_t)(NS + 3)*cap + w];
-      R.e = b.rec[(int64_t)(NS + 5)*cap + w];
-      R.rho = b.rec[(int64_t)(NS + 6)*cap + w];
-      R.dpde = b.rec[(int64_t)(NS + 7)*cap + w];
-      R.a2 = b.rec[(int64_t)(2*NS + 8)*cap + w];
       typename E_t::Proj J;
-      E_t::proj(J, R);
-      // weights of the species sums of the left-eigenvector products
-      // (rhs.inl:443-451)
-      double wj[NS];
 #pragma unroll
-      for (int j = 0; j < NS; j++) wj[j] = (J.Coeff - b.rec[(int64_t)(NS + 8 + j)*cap + w])*J.iaRoe2;
-      for (int i = 0; i < NEQ; i++) {
-         if (owner(i) != wv) continue;             // uniform
-         // the point values are re-read from LDS and the species sums
-         // re-formed for every component: held in registers across the
-         // loop they would cost some 120 VGPRs
+      for (int j = 0; j < 3; j++) R.v[j] = b.rec[(int64_t)(NS + j)*cap + wr];
+      R.a = b.rec[(int64_t)(NS + 3)*cap + wr];
+      R.e = b.rec[(int64_t)(NS + 5)*cap + wr];
+      R.rho = b.rec[(int64_t)(NS + 6)*cap + wr];
+      R.dpde = b.rec[(int64_t)(NS + 7)*cap + wr];
+      R.a2 = b.rec[(int64_t)(2*NS + 8)*cap + wr];
+      double dpdrhoi[NS];
+#pragma unroll
+      for (int j = 0; j < NS; j++) dpdrhoi[j] = b.rec[(int64_t)(NS + 8 + j)*cap + wr];
+      for (int k = wv; k < 6; k += TENO_WAVES) {
+         const int off = (k == 2) ? 0 : c_st.Cp[t][k - (k > 2 ? 1 : 0)];
+         const P3 P = wplus(g, DIR, q, off);
+         double pv[NS + 6];
+#pragma unroll
+         for (int v = 0; v < NS + 6; v++)
+            pv[v] = (v < NS + 4) ? ld<double>(f.Conserved, P, v)
+                  : (v == NS + 4) ? ld<double>(f.velocity, P, iN) : ld<double>(f.pressure, P);
+         if (k == wv) E_t::proj(J, R);
+         double (*pt)[64] = &S.pt[k*NPV];
+         double s1q = 0.0, sqq = 0.0, s1f = 0.0, sqf = 0.0;
+#pragma unroll
+         for (int j = 0; j < NS; j++) {
+            const double wj = (J.Coeff - dpdrhoi[j])*J.iaRoe2;
+            s1q += wj*pv[j];
+            sqq += pv[j];
+            const double fq = pv[j]*pv[St::UN];
+            s1f += wj*fq;
+            sqf += fq;
+         }
+#pragma unroll
+         for (int v = 0; v < NS + 6; v++) pt[v][lane] = pv[v];
+         pt[St::S1Q][lane] = s1q;
+         pt[St::SQQ][lane] = sqq;
+         pt[St::S1F][lane] = s1f;
+         pt[St::SQF][lane] = sqf;
+      }
+      __syncthreads();
+      const bool all_std = __ballot(t != Std_node) == 0ull;
+      for (int i = wv; i < NEQ; i += TENO_WAVES) {
+         // the point values are re-read from LDS for every component
          asm volatile("" ::: "memory");
-         const double lam = b.rec[(int64_t)(2*NS + ((i == 0) ? 9 : (i == NEQ-1) ? 11 : 10))*cap + w];
-         const double Ysel = (i >= 1 && i <= NS) ? b.rec[(int64_t)(i - 1)*cap + w] : 0.0;
+         const double lam = b.rec[(int64_t)(2*NS + ((i == 0) ? 9 : (i == NEQ-1) ? 11 : 10))*cap + wr];
+         const double Ysel = (i >= 1 && i <= NS) ? b.rec[(int64_t)(i - 1)*cap + wr] : 0.0;
          double vp[6], vm[6];
 #pragma unroll
          for (int k = 0; k < 6; k++) {
-            const double un = S.pt[k*NPV + NS + 4][lane];
-            const double pr = S.pt[k*NPV + NS + 5][lane];
-            double s1q = 0.0, sqq = 0.0, s1f = 0.0, sqf = 0.0, qs = 0.0;
-#pragma unroll
-            for (int j = 0; j < NS; j++) {
-               const double qv = S.pt[k*NPV + j][lane];
-               if (j == i - 1) qs = qv;
-               s1q += wj[j]*qv;
-               sqq += qv;
-               const double fq = qv*un;
-               s1f += wj[j]*fq;
-               sqf += fq;
-            }
+            const double (*pt)[64] = &S.pt[k*NPV];
+            const double un = pt[St::UN][lane], pr = pt[St::PR][lane];
+            const double qs = (i >= 1 && i <= NS) ? pt[i - 1][lane] : 0.0;
             double qm[4], fm[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) { qm[j] = S.pt[k*NPV + NS + j][lane]; fm[j] = qm[j]*un; }
+            for (int j = 0; j < 4; j++) { qm[j] = pt[NS + j][lane]; fm[j] = qm[j]*un; }
             fm[iN] += pr;
             fm[3] += pr*un;
-            const double Q = E_t::char_row(i, R, J, s1q, sqq, qs, qm, Ysel);
-            const double Fv = E_t::char_row(i, R, J, s1f, sqf, qs*un, fm, Ysel);
+            const double Q = E_t::char_row(i, R, J, pt[St::S1Q][lane], pt[St::SQQ][lane], qs, qm, Ysel);
+            const double Fv = E_t::char_row(i, R, J, pt[St::S1F][lane], pt[St::SQF][lane], qs*un, fm, Ysel);
             vp[k] = Fv + lam*Q;
             vm[k] = Fv - lam*Q;
          }
          uint32_t bp, bm;
          double FPlus, FMinus;
-         if (OP != 1 && all_std) {
-            FPlus  = teno_reconstruct<OP, 0, true>(vp, tt, &bp);
-            FMinus = teno_reconstruct<OP, 1, true>(vm, tt, &bm);
+         if (all_std) {
+            FPlus  = teno_reconstruct<OP, 0, true>(vp, t, &bp, S.w);
+            FMinus = teno_reconstruct<OP, 1, true>(vm, t, &bm, S.w);
          } else {
-            FPlus  = teno_reconstruct<OP, 0>(vp, tt, &bp);
-            FMinus = teno_reconstruct<OP, 1>(vm, tt, &bm);
+            FPlus  = teno_reconstruct<OP, 0>(vp, t, &bp, S.w);
+            FMinus = teno_reconstruct<OP, 1>(vm, t, &bm, S.w);
          }
-         S.fc[bb][i][lane] = -0.5*(FPlus + FMinus);
-         S.bits[bb][i][lane] = (uint8_t)(bp | (bm << 4));
-      }
-   };
-
-   // The two roles run their own loops (wave-uniform branch), so that the
-   // loader's gathered values are not live across the component code; both
-   // loops reach the same 1 + 2K barriers.  Wave 0 also back-projects the
-   // previous chunk before its components (held next to the gathered values
-   // in the loader, the back-projection's registers would double its
-   // footprint).
-   if (K == 0) return;                          // uniform over the block
-   if (wv == LOADER) {
-      {
-         double pv[6*NPV];
-         uint32_t fi;
-         int ti;
-         gather(chunk(0), pv, fi, ti);
-         hand_over(pv, fi, ti, 0);
+         S.fc[i][lane] = -0.5*(FPlus + FMinus);
+         S.bits[i][lane] = (uint8_t)(bp | (bm << 4));
       }
       __syncthreads();
-      for (uint32_t k = 0; k < K; k++) {
-         double pv[6*NPV];                      // live from the gather to the hand-over only
-         uint32_t fi = 0;
-         int ti = 0;
-         if (k + 1 < K) gather(chunk(k + 1), pv, fi, ti);
-         __syncthreads();                       // chunk k's components are in LDS, its point values are free
-         if (k + 1 < K) hand_over(pv, fi, ti, (int)((k + 1u) & 1u));
-         __syncthreads();                       // chunk k + 1's point values are in LDS
-      }
-   } else {
-      __syncthreads();
-      for (uint32_t k = 0; k < K; k++) {
-         if (wv == 0 && k > 0) finish(chunk(k - 1), (int)((k - 1u) & 1u));
-         components(chunk(k), (int)(k & 1u));
-         __syncthreads();
-         __syncthreads();
-      }
-      if (wv == 0) finish(chunk(K - 1), (int)((K - 1u) & 1u));
    }
+   if (wv == LAST) finish(L + (nchunks - 1u - L)/gridDim.x*gridDim.x);
 }
 
 template<class MX, int DIR, bool LISTED>

@@ -91,29 +91,87 @@ __device__ __forceinline__ void smooth_minus(const double *v, double *s)
    s[3] = C14*a1*a1 + C24*a2*a2 + C34*a3*a3;
 }
 
+// 1/d to within a rounding, for quantities that only enter a stencil
+// selection (see ipow6): the hardware's estimate (2^-24) and one third-order
+// correction, 4 instructions against the 11 of a division
+__device__ __forceinline__ double sel_rcp(double d)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+   const double r = __builtin_amdgcn_rcp(d);
+   const double e = fma(-d, r, 1.0);
+   return fma(r, fma(e, e, e), r);
+#else
+   return 1.0/d;
+#endif
+}
+
+// Normalised weights of the interior node type for the 16 selections: a
+// reconstruction reads its four from LDS instead of forming them (a division,
+// three sums and eight products)
+struct StdWeights { double w[16][4]; };
+constexpr StdWeights make_std_weights()
+{
+   StdWeights t = {};
+   for (int s = 1; s < 16; s++) {
+      double w[4] = {};
+      for (int k = 0; k < 4; k++) w[k] = rows::std4[k]*(s >> k & 1);
+      const double an = 1.0/(w[0] + w[1] + w[2] + w[3]);
+      for (int k = 0; k < 4; k++) t.w[s][k] = w[k]*an;
+   }
+   return t;
+}
+__constant__ constexpr StdWeights c_stdw = make_std_weights();
+
+// The interior candidates of v less base, in the order of the general row
+// product but without its zero entries: a zero times a finite value adds
+// nothing to the sum, and what it does with a value that is not finite is
+// restored by the caller
+template<int SIDE>
+__device__ __forceinline__ void std_candidates(const double *v, double base, double *var)
+{
+   using namespace rows;
+   const double a = v[1]*s1p[1] + v[2]*s1p[2] + v[3]*s1p[3] - base;
+   const double b = v[2]*s2p[2] + v[3]*s2p[3] + v[4]*s2p[4] - base;
+   var[0] = SIDE ? b : a;
+   var[1] = SIDE ? a : b;
+   if (SIDE) {
+      var[2] = v[3]*s3m[3] + v[4]*s3m[4] + v[5]*s3m[5] - base;
+      var[3] = v[0]*s4m[0] + v[1]*s4m[1] + v[2]*s4m[2] + v[3]*s4m[3] - base;
+   } else {
+      var[2] = v[0]*s3p[0] + v[1]*s3p[1] + v[2]*s3p[2] - base;
+      var[3] = v[2]*s4p[2] + v[3]*s4p[3] + v[4]*s4p[4] + v[5]*s4p[5] - base;
+   }
+}
+
 // OP 0: TENO_Op<-10>, 1: TENOA_Op<-8>, 2: TENOLAD_Op<-16>; SIDE 0 plus, 1 minus.
 // Returns the reconstructed value; *bits receives b1 | b2<<1 | b3<<2 | b4<<3.
-// STD: the caller guarantees t == Std_node; the stencil rows and weights are
-// then immediates instead of per-lane table loads.
+// STD: the caller guarantees t == Std_node; the stencil rows are then
+// immediates and the weights come from wtab (StdWeights in LDS) instead of
+// per-lane table loads.
+// The smoothness ratios, their sixth powers and the cut-off only select; the
+// value depends on the selected stencils alone.  The selection a_k/sum < cut
+// is therefore formed as a_k < cut*sum, and the ratios from sel_rcp: of the
+// seven divisions of a reconstruction (77 of its some 200 FP64 instructions)
+// none is left on the interior path.
 template<int OP, int SIDE, bool STD = false>
-__device__ __forceinline__ double teno_reconstruct(const double *v, int t, uint32_t *bits)
+__device__ __forceinline__ double teno_reconstruct(const double *v, int t, uint32_t *bits, const double (*wtab)[4])
 {
    const double *Coeffs = STD ? rows::std4 : SIDE ? c_st.CoeffM[t] : c_st.CoeffP[t];
-   const double *const std_rows[4] = { SIDE ? rows::s2p : rows::s1p, SIDE ? rows::s1p : rows::s2p,
-                                       SIDE ? rows::s3m : rows::s3p, SIDE ? rows::s4m : rows::s4p };
    const double *Recon  = SIDE ? c_st.ReconM[t] : c_st.ReconP[t];
    if (STD) t = Std_node;
    double s[4];
    if (SIDE) smooth_minus(v, s); else smooth_plus(v, s);
    const double eps = (OP == 0) ? ten_pow_chain(-10) : (OP == 1) ? ten_pow_chain(-8) : ten_pow_chain(-16);
-   const double tau6 = fabs(s[3] - (s[2] + s[1] + 4*s[0])/6);
+   const double tau6 = fabs(s[3] - (s[2] + s[1] + 4*s[0])*(1.0/6.0));
    double chi[4], a[4];
 #pragma unroll
-   for (int k = 0; k < 4; k++) { chi[k] = tau6/(s[k] + eps); a[k] = ipow6(1 + chi[k]); }
-   double cut;
-   if (OP == 0) {
+   for (int k = 0; k < 4; k++) { chi[k] = tau6*sel_rcp(s[k] + eps); a[k] = ipow6(1 + chi[k]); }
+   if (!STD && (OP != 1 || t != Std_node)) {
 #pragma unroll
       for (int k = 0; k < 4; k++) if (Coeffs[k] < 1e-10) a[k] = 0.0;
+   }
+   double cut;
+   if (OP == 0) {
       cut = 1e-6;
    } else if (OP == 1) {
       if (t == Std_node) {
@@ -121,50 +179,56 @@ __device__ __forceinline__ double teno_reconstruct(const double *v, int t, uint3
          const double Ren_eps = 0.9*Ren_r_c*1e-16/(1.0 - 0.9*Ren_r_c);
          const double Ren_irc = 1.0/Ren_r_c;
          const double Smooth_pow = 9.5, Shock_pow = 6.0, Diff_pow = Smooth_pow - Shock_pow;
-         const double var2 = fabs(v[1] - v[0]);
-         const double var3 = fabs(v[2] - v[1]);
-         const double var4 = fabs(v[3] - v[2]);
-         const double var5 = fabs(v[4] - v[3]);
-         const double var6 = fabs(v[5] - v[4]);
-         double eta = dmin((2*var2*var3 + Ren_eps)/(var2*var2 + var3*var3 + Ren_eps),
-                           (2*var3*var4 + Ren_eps)/(var3*var3 + var4*var4 + Ren_eps));
-         eta = dmin(eta,   (2*var4*var5 + Ren_eps)/(var4*var4 + var5*var5 + Ren_eps));
-         eta = dmin(eta,   (2*var5*var6 + Ren_eps)/(var5*var5 + var6*var6 + Ren_eps));
+         double var[5], sq[5];
+#pragma unroll
+         for (int k = 0; k < 5; k++) { var[k] = fabs(v[k+1] - v[k]); sq[k] = var[k]*var[k]; }
+         double eta = 0.0;
+#pragma unroll
+         for (int k = 0; k < 4; k++) {
+            const double r = (2*var[k]*var[k+1] + Ren_eps)*sel_rcp(sq[k] + sq[k+1] + Ren_eps);
+            eta = k ? dmin(eta, r) : r;
+         }
          const double delta = 1 - dmin(eta*Ren_irc, 1.0);
          const double decay = ipow4(1 - delta)*(1 + 4*delta);
          const int power = min(max((int)floor(Smooth_pow - Diff_pow*(1 - decay)), 0), 13);
          cut = (double)c_st.p10[power];
       } else {
-#pragma unroll
-         for (int k = 0; k < 4; k++) if (Coeffs[k] < 1e-10) a[k] = 0.0;
          cut = (double)c_st.p10[4];
       }
    } else {
-#pragma unroll
-      for (int k = 0; k < 4; k++) if (Coeffs[k] < 1e-10) a[k] = 0.0;
       const double Smooth_pow = 12.5, Shock_pow = 3.0, iH = 1e-1, Diff_pow = Smooth_pow - Shock_pow;
       const double chiMax = dmax(chi[0], dmax(chi[1], dmax(chi[2], chi[3])));
-      const double theta = 1.0/(1 + chiMax*iH);
+      const double theta = sel_rcp(1 + chiMax*iH);
       const int power = min(max((int)floor(Shock_pow + Diff_pow*theta), 0), 13);
       cut = (double)c_st.p10[power];
    }
-   double an = 1.0/(a[0] + a[1] + a[2] + a[3]);
+   const double lim = cut*(a[0] + a[1] + a[2] + a[3]);
    int b[4];
 #pragma unroll
-   for (int k = 0; k < 4; k++) b[k] = (a[k]*an < cut) ? 0 : 1;
-   *bits = (uint32_t)(b[0] | b[1] << 1 | b[2] << 2 | b[3] << 3);
+   for (int k = 0; k < 4; k++) b[k] = (a[k] < lim) ? 0 : 1;
+   const uint32_t sel = (uint32_t)(b[0] | b[1] << 1 | b[2] << 2 | b[3] << 3);
+   *bits = sel;
    const double base = SIDE ? v[3] : v[2];
    double var[4], w[4];
+   if (STD) {
+      std_candidates<SIDE>(v, base, var);
 #pragma unroll
-   for (int k = 0; k < 4; k++) {
-      const double *R = STD ? std_rows[k] : &Recon[6*k];
-      var[k] = v[0]*R[0] + v[1]*R[1] + v[2]*R[2] + v[3]*R[3] + v[4]*R[4] + v[5]*R[5] - base;
-      w[k] = Coeffs[k]*b[k];
+      for (int k = 0; k < 4; k++) w[k] = wtab[sel][k];
+      // var[2] and var[3] together hold every value of the stencil: not a
+      // number if one of them is not finite, as with the zero entries
+      return base + w[0]*var[0] + w[1]*var[1] + w[2]*var[2] + w[3]*var[3] + 0.0*(var[2] + var[3]);
+   } else {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+         const double *R = &Recon[6*k];
+         var[k] = v[0]*R[0] + v[1]*R[1] + v[2]*R[2] + v[3]*R[3] + v[4]*R[4] + v[5]*R[5] - base;
+         w[k] = Coeffs[k]*b[k];
+      }
+      const double an = 1.0/(w[0] + w[1] + w[2] + w[3]);
+#pragma unroll
+      for (int k = 0; k < 4; k++) w[k] = w[k]*an;
+      return base + w[0]*var[0] + w[1]*var[1] + w[2]*var[2] + w[3]*var[3];
    }
-   an = 1.0/(w[0] + w[1] + w[2] + w[3]);
-#pragma unroll
-   for (int k = 0; k < 4; k++) w[k] = w[k]*an;
-   return base + w[0]*var[0] + w[1]*var[1] + w[2]*var[2] + w[3]*var[3];
 }
 
 // TENOsensor::TENOA (metric.inl:352-403): true = smooth
