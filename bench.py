@@ -37,11 +37,9 @@ RHS_BYTES_PER_CELL = 495.0
 # Per-kernel algorithmic bytes per unit (AirMix, NS = 5, nEq = 9); the unit
 # count of one launch comes from the workload (cells, faces, TENO faces).
 #   euler_classify  per face: nType + own-cell sensor (5 B) read
-#   euler_kg_species per cell (KG walk, species group): rho, u_n, Y 5 (56 B)
-#                   + nType + sensor (5 B) + m_e (8 B) read, Conserved_t[0:5]
-#                   read-modify-write (80 B) = 149 B
-#   euler_kg_flow   per cell (KG walk, momentum/energy group): rho, u 3, H,
-#                   p (48 B) + 13 B as above, Conserved_t[5:9] RMW (64 B) = 125 B
+#   euler_kg        per cell, three directions: rho, u 3, H, p, Y 5 (88 B),
+#                   nType, sensor and m_e of each direction (39 B) read,
+#                   Conserved_t read-modify-write (144 B) = 271 B
 #   euler_roe       per TENO face: own-cell Roe inputs (88 B) + SoS (8 B)
 #                   read, face record (22 doubles, 176 B) written = 272 B
 #   euler_teno      per TENO face: face record (21 doubles, 168 B) read, the
@@ -51,19 +49,15 @@ RHS_BYTES_PER_CELL = 495.0
 #                   not counted; FP64-bound, see KERNEL_FLOPS
 #   euler_divergence per cell: face flux 72 B + m_e 8 B read, Conserved_t
 #                   read-modify-write 144 B = 224 B
-#   diffusion_species per cell: rho Y 5, T, X 5, rho, lambda, D 5, m_s, m_d
-#                   (20 doubles) + nType read, heat flux per face written,
-#                   Conserved_t[0:5] read-modify-write (80 B) = 252 B
-#   diffusion_stress per cell: mu, u 3, m_s, m_d and the transverse m_d 2
-#                   (8 doubles) + 3 node types + heat flux read,
-#                   Conserved_t[5:9] RMW (64 B) = 148 B
+#   diffusion       per cell, three directions: rho Y 5, T, X 5, rho, lambda,
+#                   D 5, mu, u 3 (176 B), m_s, m_d and nType of each direction
+#                   (60 B) read, Conserved_t read-modify-write (144 B) = 380 B
 #   chem_source     per cell: rho, p, T, Y 5 (64 B) read, Conserved_t (9
 #                   doubles, 72 B) written = 136 B (the source also clears
 #                   the stage's Conserved_t)
 #   enthalpy        per cell: rhoE, p, rho read, H written = 32 B
-KERNEL_BYTES = {"euler_classify": 5.0, "euler_kg_species": 149.0, "euler_kg_flow": 125.0, "euler_roe": 272.0,
-                "euler_teno": 416.0, "euler_divergence": 224.0, "diffusion_species": 252.0,
-                "diffusion_stress": 148.0, "chem_source_kernel": 136.0, "enthalpy": 32.0}
+KERNEL_BYTES = {"euler_classify": 5.0, "euler_kg": 271.0, "euler_roe": 272.0, "euler_teno": 416.0,
+                "euler_divergence": 224.0, "diffusion": 380.0, "chem_source_kernel": 136.0, "enthalpy": 32.0}
 # FP64 operations per unit of the compute-bound kernels (hand count of the
 # source, FMA-free build: per component the species sums and split fluxes of
 # six points ~600, two TENO reconstructions ~300; nine components plus the

@@ -321,7 +321,7 @@ static int64_t gcd64(int64_t a, int64_t b) { while (b) { const int64_t t = a % b
 struct LayoutCheck {
    int64_t bsz[3];
    int64_t base[3];
-   bool have = false;
+   bool have = false, soa = true;
    const char *first = "";
    int add(htr_view &v, int esize, const char *name, const int64_t *blo)
    {
@@ -334,6 +334,7 @@ struct LayoutCheck {
          k = gcd64(k, s[d]);
       }
       if (k == 0) k = 1;
+      soa = soa && k == 1;
       int64_t b[3];
       for (int d = 0; d < 3; d++) b[d] = s[d]/k;
       if (!have) {
@@ -396,6 +397,7 @@ static int layout_views(const htr_grid *g, htr_fields &out, htr_view *extra, int
       if (rc) return rc;
    }
    for (int d = 0; d < 3; d++) geo.cb[d] = (uint32_t)(L.have ? L.base[d] : 0);
+   geo.soa = L.soa ? 1 : 0;
    return HTR_OK;
 }
 
@@ -438,7 +440,6 @@ struct RhsAux {
    hipStream_t ts[3] = {};
    hipEvent_t  h = nullptr;           // caller stream: total enthalpy formed
    hipEvent_t  teno[3] = {};          // side stream d: TENO faces of direction d formed
-   hipEvent_t  used[3] = {};          // caller stream: the walks of direction d have read them
 };
 static std::map<std::pair<int, uintptr_t>, RhsAux*> g_aux;
 static int g_overlap = 0;
@@ -454,8 +455,7 @@ static RhsAux *rhs_aux(hipStream_t s)
    bool ok = hipEventCreateWithFlags(&n->h, hipEventDisableTiming) == hipSuccess;
    for (int d = 0; d < 3 && ok; d++)
       ok = hipStreamCreateWithFlags(&n->ts[d], hipStreamNonBlocking) == hipSuccess &&
-           hipEventCreateWithFlags(&n->teno[d], hipEventDisableTiming) == hipSuccess &&
-           hipEventCreateWithFlags(&n->used[d], hipEventDisableTiming) == hipSuccess;
+           hipEventCreateWithFlags(&n->teno[d], hipEventDisableTiming) == hipSuccess;
    if (!ok) {
       set_error(HTR_E_DEVICE, "side stream creation failed");
       return nullptr;
@@ -466,10 +466,10 @@ static RhsAux *rhs_aux(hipStream_t s)
 
 // The hybrid Euler sweeps with each direction's TENO passes on a side stream:
 // total enthalpy (caller stream), then the TENO passes of z, y, x on their
-// side streams, overlapping the chemistry source and the earlier directions'
-// KG walks on the caller stream; each walk waits for its direction's TENO
-// faces.  Conserved_t receives its terms in the same order as without
-// overlap (source, Euler z, y, x), so the result is the same to the bit.
+// side streams, overlapping the chemistry source on the caller stream; the KG
+// pass waits for the TENO faces of all three.  Conserved_t receives its terms
+// in the same order as without overlap (source, Euler z, y, x), so the result
+// is the same to the bit.
 template<class MX>
 static int euler_overlapped(const htr_fields &fr, const htr_mix *m, const Geo &geo, double RK0, double RK1,
                             const DtArg &dt, const htr_view &dec, int chem_source, hipStream_t s)
@@ -480,21 +480,17 @@ static int euler_overlapped(const htr_fields &fr, const htr_mix *m, const Geo &g
    if (rc) return rc;
    if (hipEventRecord(aux->h, s) != hipSuccess) return set_error(HTR_E_DEVICE, "event record failed");
    for (int d = 2; d >= 0; d--) {
-      if (hipStreamWaitEvent(aux->ts[d], aux->h, 0) != hipSuccess ||
-          hipStreamWaitEvent(aux->ts[d], aux->used[d], 0) != hipSuccess)
+      if (hipStreamWaitEvent(aux->ts[d], aux->h, 0) != hipSuccess)
          return set_error(HTR_E_DEVICE, "stream wait failed");
-      if ((rc = hybrid_part_dispatch<MX>(d, 0, fr, m->dev, geo, RK0, RK1, dt, dec, aux->ts[d], s, s))) return rc;
+      if ((rc = rhs_euler_part<MX>(d, 0, HTR_EULER_HYBRID, fr, m->dev, geo, RK0, RK1, dt, dec, aux->ts[d], s))) return rc;
       if (hipEventRecord(aux->teno[d], aux->ts[d]) != hipSuccess) return set_error(HTR_E_DEVICE, "event record failed");
    }
    if (chem_source && !m->host.constprop) rc = chem_source_launch<MixAir>(fr, m->dev, geo, s, true);
    else                                   rc = zero_rhs_launch(fr, geo, m->host.nSpec + 4, s);
    if (rc) return rc;
-   for (int d = 2; d >= 0; d--) {
+   for (int d = 2; d >= 0; d--)
       if (hipStreamWaitEvent(s, aux->teno[d], 0) != hipSuccess) return set_error(HTR_E_DEVICE, "stream wait failed");
-      if ((rc = hybrid_part_dispatch<MX>(d, 1, fr, m->dev, geo, RK0, RK1, dt, dec, aux->ts[d], s, s))) return rc;
-      if (hipEventRecord(aux->used[d], s) != hipSuccess) return set_error(HTR_E_DEVICE, "event record failed");
-   }
-   return HTR_OK;
+   return rhs_euler_part<MX>(0, 1, HTR_EULER_HYBRID, fr, m->dev, geo, RK0, RK1, dt, dec, s, s);
 }
 
 } // namespace htr
@@ -839,15 +835,24 @@ int htr_max_mach(int dir, const htr_grid *g, const htr_fields *f, double *out, v
    return done(max_mach_launch(dir, fr, geo, out, (hipStream_t)stream));
 }
 
-int htr_diffusion_flux(int dir, const htr_grid *g, const htr_fields *f, const htr_mix *m, void *stream)
+// dirs: one direction's bit, or 7
+static int diffusion(int dirs, const htr_grid *g, const htr_fields *f, const htr_mix *m, void *stream)
 {
    Geo geo; htr_fields fr; int rc = prep(g, f, m, fr, geo); if (rc) return done(rc);
-   if (dir < 0 || dir > 2) return set_error(HTR_E_ARG, "bad direction %d", dir);
    HTR_NEED(Conserved); HTR_NEED(temperature); HTR_NEED(MolarFracs); HTR_NEED(rho); HTR_NEED(mu);
    HTR_NEED(lam); HTR_NEED(Di); HTR_NEED(velocity); HTR_NEED(Conserved_t);
    for (int d = 0; d < 3; d++) { HTR_NEED(nType[d]); HTR_NEED(m_d[d]); }
-   HTR_NEED(m_s[dir]);
-   HTR_DISPATCH3(diffusion_dispatch, dir, fr, m->dev, geo, (hipStream_t)stream);
+   for (int d = 2; d >= 0; d--) if (dirs >> d & 1) HTR_NEED(m_s[d]);
+   HTR_DISPATCH3(diffusion_dispatch, dirs, fr, m->dev, geo, (hipStream_t)stream);
+}
+
+int htr_diffusion_flux(int dir, const htr_grid *g, const htr_fields *f, const htr_mix *m, void *stream)
+{
+   if (dir < 0 || dir > 2) {
+      Geo geo; htr_fields fr; const int rc = prep(g, f, m, fr, geo);
+      return rc ? done(rc) : set_error(HTR_E_ARG, "bad direction %d", dir);
+   }
+   return diffusion(1 << dir, g, f, m, stream);
 }
 
 int htr_chem_source(const htr_grid *g, const htr_fields *f, const htr_mix *m, void *stream)
@@ -961,7 +966,7 @@ int htr_workspace_reserve(const htr_grid *g, const htr_fields *f, const htr_mix 
       for (int d = 0; d < 3; d++) {
          Workspace *a = workspace(aux->ts[d]);
          if (!a) return HTR_E_DEVICE;
-         if ((rc = workspace_faces(*a, need.faces, need.list, need.teno))) return rc;
+         if ((rc = workspace_faces(*a, 0, need.list, need.teno))) return rc;
       }
    }
    return HTR_OK;
@@ -993,11 +998,7 @@ static int full_rhs(const htr_grid *g, const htr_fields *f, int scheme, double R
       rc = (k == K_CP) ? euler_overlapped<MixCP>(fr, m, geo, RK0, RK1, dt, dec, chem_source, s)
                        : euler_overlapped<MixAir>(fr, m, geo, RK0, RK1, dt, dec, chem_source, s);
       if (rc) return rc;
-      for (int d = 2; d >= 0; d--) {
-         rc = htr_diffusion_flux(d, g, f, m, stream);
-         if (rc) return rc;
-      }
-      return HTR_OK;
+      return diffusion(7, g, f, m, stream);
    }
    if (chem_source && !m->host.constprop) {
       HTR_NEED(pressure); HTR_NEED(temperature);
@@ -1009,16 +1010,21 @@ static int full_rhs(const htr_grid *g, const htr_fields *f, int scheme, double R
    // total enthalpy once for the three sweeps
    rc = (k == K_CP) ? enthalpy_launch<MixCP>(fr, geo, s) : enthalpy_launch<MixAir>(fr, geo, s);
    if (rc) return rc;
-   for (int d = 2; d >= 0; d--) {
-      rc = (k == K_CP) ? euler_dispatch<MixCP>(d, scheme, fr, m->dev, geo, RK0, RK1, dt, dec, s, true)
-                       : euler_dispatch<MixAir>(d, scheme, fr, m->dev, geo, RK0, RK1, dt, dec, s, true);
-      if (rc) return rc;
+   if (scheme == HTR_EULER_HYBRID || scheme == HTR_EULER_KG) {
+      for (int d = (scheme == HTR_EULER_KG) ? -1 : 2; d >= -1; d--) {
+         const int part = d < 0 ? 1 : 0;
+         rc = (k == K_CP) ? rhs_euler_part<MixCP>(d, part, scheme, fr, m->dev, geo, RK0, RK1, dt, dec, s, s)
+                          : rhs_euler_part<MixAir>(d, part, scheme, fr, m->dev, geo, RK0, RK1, dt, dec, s, s);
+         if (rc) return rc;
+      }
+   } else {
+      for (int d = 2; d >= 0; d--) {
+         rc = (k == K_CP) ? euler_dispatch<MixCP>(d, scheme, fr, m->dev, geo, RK0, RK1, dt, dec, s, true)
+                          : euler_dispatch<MixAir>(d, scheme, fr, m->dev, geo, RK0, RK1, dt, dec, s, true);
+         if (rc) return rc;
+      }
    }
-   for (int d = 2; d >= 0; d--) {
-      rc = htr_diffusion_flux(d, g, f, m, stream);
-      if (rc) return rc;
-   }
-   return HTR_OK;
+   return diffusion(7, g, f, m, stream);
 }
 
 int htr_full_rhs(const htr_grid *g, const htr_fields *f, int scheme, double RK0, double RK1,

@@ -1,411 +1,337 @@
 // diffusion.hip -- viscous, heat and multicomponent (Fick + correction
-// velocity) flux divergence along one direction.
+// velocity) flux divergence.
 //
 // Reference: src/prometeo_rhs.inl:1058-1282 (GetSigma, GetDiffusionFlux,
-// updateRHSSpan), src/prometeo_rhs.cu:461-622.  One pass per direction:
-// line segments walked face by face, the divergence fused (below).
+// updateRHSSpan), src/prometeo_rhs.cu:461-622.  One thread per cell forms both
+// its faces along every direction of the launch and adds (F+ - F-) m_d to
+// Conserved_t, which is read and written once for all directions.
+//
+// Each face is thus formed twice, which costs 1400 FP64 operations more per
+// cell and saves two thirds of the passes over memory: the walks along the
+// lines that this replaces took a pass per direction and component group
+// (species; momentum and energy, with the heat flux handed over through a
+// buffer), each reading its fields and reading and writing Conserved_t.  Bound
+// by the loads' address cycles (16 per 64-lane 8-byte load, 270 loads per
+// cell) and FP64 issue at two waves per SIMD.  All three directions, with the
+// walks in brackets: 256^3 air 3.8 (4.8) ms, 512x256x128 boundary layer 3.8
+// (4.8) ms, 117x93x75 air 195 (315) us, 32^3 one species 13 (102) us.
 #include "common.hpp"
 #include "kernels.hpp"
-#include <type_traits>
 
 namespace htr {
 
-template<class MX, int DIR>
-struct Diffusion {
-   static constexpr int NS = MX::NS, NEQ = MX::NEQ;
+// weights of the left and right cell of a face (Interp2Staggered)
+struct FaceW {
+   double a, b;
+   __device__ double operator()(double l, double r) const { return a*l + b*r; }
+};
+
+template<class MX, bool SOA>
+struct DiffCell {
+   static constexpr int NS = MX::NS;
+   // what the species part of a face reads of a cell
+   double X[NS], Di[NS], rY[NS];
+   double rho, T, lam, W;      // W: molar weight of the mixture from X
+   __device__ __forceinline__ void load(const htr_fields &f, const DMix &m, uint32_t o)
+   {
+#pragma unroll
+      for (int i = 0; i < NS; i++) {
+         X[i] = ldo<double, SOA>(f.MolarFracs, o, i);
+         Di[i] = ldo<double, SOA>(f.Di, o, i);
+         rY[i] = ldo<double, SOA>(f.Conserved, o, i);
+      }
+      rho = ldo<double, SOA>(f.rho, o);
+      T = ldo<double, SOA>(f.temperature, o);
+      lam = ldo<double, SOA>(f.lam, o);
+      W = MX::MolarWeightFromX(m, X);
+   }
+};
+
+// GetDiffusionFlux (rhs.inl:1140-1218) at the face between cells P and Q,
+// species part: the species fluxes into Flux[0..NS-1] and the heat flux
+// (conduction + species enthalpy transport) returned
+template<class MX, bool SOA>
+__device__ __forceinline__ double species_face(double *Flux, const DMix &m, const FaceW &w, double m_s,
+                                               const DiffCell<MX, SOA> &P, const DiffCell<MX, SOA> &Q)
+{
+   constexpr int NS = MX::NS;
+   const double rho_s = w(P.rho, Q.rho);
+   const double iMixW_s = 1.0/w(P.W, Q.W);
+   const double T_s = w(P.T, Q.T);
+   double heatFlux = w(P.lam, Q.lam)*m_s*(P.T - Q.T);
+   double ViCorr = 0.0;
+   double hs[NS];
+   MX::SpeciesEnthalpies(m, hs, T_s);
+#pragma unroll
+   for (int i = 0; i < NS; i++) {
+      const double YiVi = w(P.Di[i], Q.Di[i])*m_s*(P.X[i] - Q.X[i])*MX::SpeciesW(m, i)*iMixW_s;
+      Flux[i] = -rho_s*YiVi;
+      heatFlux += rho_s*YiVi*hs[i];
+      ViCorr += YiVi;
+   }
+#pragma unroll
+   for (int i = 0; i < NS; i++) {
+      const double corr = w(P.rY[i], Q.rY[i])*ViCorr;
+      Flux[i] += corr;
+      heatFlux -= corr*hs[i];
+   }
+   return heatFlux;
+}
+
+// The transverse gradients that the stress of a face along DIR takes from one
+// of its cells: along D1 of velocity components (A1, B1), along D2 of (A2, B2)
+template<int DIR>
+struct Transverse {
    static constexpr int D1 = (DIR == 0) ? 1 : 0;   // getT1
    static constexpr int D2 = (DIR == 2) ? 1 : 2;   // getT2
+   static constexpr int A1 = 0, B1 = (DIR == 2) ? 2 : 1;
+   static constexpr int A2 = (DIR == 0) ? 0 : 1, B2 = 2;
+   double a1, b1, a2, b2;
+};
+
+// momentum part of a face: the viscous stress into s and u.sigma returned
+// (GetSigma, rhs.inl:1058-1137)
+template<int DIR>
+__device__ __forceinline__ double stress_face(double *s, const FaceW &w, double m_s, const double *vp, const double *vq,
+                                              double muP, double muQ, const Transverse<DIR> &L, const Transverse<DIR> &R)
+{
+   const double mu_s = w(muP, muQ);
+   double dn[3];
+#pragma unroll
+   for (int i = 0; i < 3; i++) dn[i] = m_s*(vq[i] - vp[i]);
+   const double a1 = w(L.a1, R.a1), b1 = w(L.b1, R.b1), a2 = w(L.a2, R.a2), b2 = w(L.b2, R.b2);
+   if (DIR == 0) {             // dU/dy, dV/dy, dU/dz, dW/dz
+      s[0] = mu_s*(4*dn[0] - 2*b1 - 2*b2)/3;
+      s[1] = mu_s*(dn[1] + a1);
+      s[2] = mu_s*(dn[2] + a2);
+   } else if (DIR == 1) {      // dU/dx, dV/dx, dV/dz, dW/dz
+      s[0] = mu_s*(dn[0] + b1);
+      s[1] = mu_s*(4*dn[1] - 2*a1 - 2*b2)/3;
+      s[2] = mu_s*(dn[2] + a2);
+   } else {                    // dU/dx, dW/dx, dV/dy, dW/dy
+      s[0] = mu_s*(dn[0] + b1);
+      s[1] = mu_s*(dn[1] + b2);
+      s[2] = mu_s*(4*dn[2] - 2*a1 - 2*a2)/3;
+   }
+   double uSigma = 0.0;
+#pragma unroll
+   for (int i = 0; i < 3; i++) uSigma += w(vp[i], vq[i])*s[i];
+   return uSigma;
+}
+
+// The thread's cell, its neighbours and the faces' node types and metrics
+template<class MX, int DIRS, bool SOA>
+struct Diffusion {
+   static constexpr int NS = MX::NS, NEQ = MX::NEQ;
+   using Cell = DiffCell<MX, SOA>;
    const htr_fields &f;
    const DMix &m;
    const Geo &g;
+   const P3 &p;
+   uint32_t up[3], dn[3];      // offsets to the next and the previous cell along a direction
 
-   __device__ double vel(const P3 &p, int i) const { return ld<double>(f.velocity, p, i); }
+   __device__ __forceinline__ Diffusion(const htr_fields &f_, const DMix &m_, const Geo &g_, const P3 &p_)
+      : f(f_), m(m_), g(g_), p(p_)
+   {
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+         int c = p.c[d];
+         uint32_t o = p.o;
+         step_up(g, d, c, o);
+         up[d] = o - p.o;
+         c = p.c[d];
+         o = p.o;
+         step_down(g, d, c, o);
+         dn[d] = o - p.o;
+      }
+   }
 
+   // the two faces of the cell along DIR: interpolation weights and staggered
+   // metric of their left cells.  The minus face of a line's first cell is
+   // that of p + offM1(nType) (rhs.inl:1253-1254): the previous cell's, but the
+   // cell's own (plus) face at a left boundary node.
+   // next: the cell after such a first cell, whose minus face is that plus face.
+   struct Faces2 { FaceW wp, wm; double msp, msm, md; bool own, next; };
+   template<int DIR>
+   __device__ __forceinline__ Faces2 faces() const
+   {
+      const uint32_t om = p.o + dn[DIR];
+      const int t = ldo<int, SOA>(f.nType[DIR], p.o), tm = ldo<int, SOA>(f.nType[DIR], om);
+      Faces2 F;
+      F.wp = F.wm = { 0.5, 0.5 };
+      if (!wave_all(t == Std_node && tm == Std_node)) {
+         F.wp = { (double)c_st.Interp[t][0], (double)c_st.Interp[t][1] };
+         F.wm = { (double)c_st.Interp[tm][0], (double)c_st.Interp[tm][1] };
+      }
+      F.msp = ldo<double, SOA>(f.m_s[DIR], p.o);
+      F.msm = ldo<double, SOA>(f.m_s[DIR], om);
+      F.md = ldo<double, SOA>(f.m_d[DIR], p.o);
+      F.own = p.c[DIR] == g.elo[DIR] && (t == L_S_node || t == L_C_node);
+      F.next = p.c[DIR] == g.elo[DIR] + 1 && (tm == L_S_node || tm == L_C_node);
+      return F;
+   }
+
+   // species fluxes along DIR into ct[0..NS-1]; the heat fluxes of the plus and
+   // minus face into hp, hm
+   template<int DIR>
+   __device__ __forceinline__ void species(double *ct, const Cell &C0, double &hp, double &hm) const
+   {
+      const Faces2 F = faces<DIR>();
+      double Fp[NS], Fm[NS];
+      Cell C;
+      C.load(f, m, p.o + up[DIR]);
+      hp = species_face<MX, SOA>(Fp, m, F.wp, F.msp, C0, C);
+#pragma unroll
+      for (int i = 0; i < NS; i++) HTR_PIN(Fp[i]);
+      HTR_PIN(hp);
+      C.load(f, m, p.o + dn[DIR]);
+      hm = species_face<MX, SOA>(Fm, m, F.wm, F.msm, C, C0);
+      if (F.own) hm = hp;
+#pragma unroll
+      for (int i = 0; i < NS; i++) {
+         if (F.own) Fm[i] = Fp[i];
+         ct[i] += (Fp[i] - Fm[i])*F.md;
+         HTR_PIN(ct[i]);
+      }
+      HTR_PIN(hm);
+   }
+
+   __device__ double vel(uint32_t o, int i) const { return ldo<double, SOA>(f.velocity, o, i); }
+
+   // getDeriv of velocity component i along DD at the cell of offset o, whose
+   // coordinate along DD is the thread's own
+   struct Node { bool lo, hi; double g0, g1, mm; };
    template<int DD>
-   __device__ void deriv3(const P3 &p, double *out) const
+   __device__ __forceinline__ Node node(uint32_t o) const
    {
-      const int t = ld<int>(f.nType[DD], p);
-      const double mm = ld<double>(f.m_d[DD], p);
-      const P3 pM1 = wminus(g, DD, p, c_st.Cp[t][1]);
-      const P3 pP1 = wplus(g, DD, p, c_st.Cp[t][2]);
-      const double g0 = (double)c_st.Grad[t][0], g1 = (double)c_st.Grad[t][1];
+      Node n;
+      const int t = ldo<int, SOA>(f.nType[DD], o);
+      n.mm = ldo<double, SOA>(f.m_d[DD], o);
+      n.g0 = n.g1 = 0.5;
+      if (!wave_all(t == Std_node)) { n.g0 = (double)c_st.Grad[t][0]; n.g1 = (double)c_st.Grad[t][1]; }
+      // stencil offsets of a node type are 0 or the natural ones
+      n.lo = t == L_S_node || t == L_C_node;
+      n.hi = t == R_S_node || t == R_C_node;
+      return n;
+   }
+   template<int DD>
+   __device__ __forceinline__ double deriv(const Node &n, uint32_t o, int i, double x) const
+   {
+      const double a = vel(o + dn[DD], i), b = vel(o + up[DD], i);
+      return (n.g0*(x - (n.lo ? x : a)) + n.g1*((n.hi ? x : b) - x))*n.mm;
+   }
+
+   template<int DIR>
+   __device__ __forceinline__ Transverse<DIR> transverse(uint32_t o, const double *v) const
+   {
+      using T = Transverse<DIR>;
+      T r;
+      const Node n1 = node<T::D1>(o), n2 = node<T::D2>(o);
+      r.a1 = deriv<T::D1>(n1, o, T::A1, v[T::A1]);
+      r.b1 = deriv<T::D1>(n1, o, T::B1, v[T::B1]);
+      r.a2 = deriv<T::D2>(n2, o, T::A2, v[T::A2]);
+      r.b2 = deriv<T::D2>(n2, o, T::B2, v[T::B2]);
+      HTR_PIN(r.a1); HTR_PIN(r.b1); HTR_PIN(r.a2); HTR_PIN(r.b2);
+      return r;
+   }
+
+   // stress and energy fluxes along DIR into ct[0..3] (momentum, energy); v0, mu0,
+   // G0: the cell's velocity, viscosity and transverse gradients.  Where the
+   // minus face is the plus face, the reference takes the plus face's left
+   // gradients at p + 1, handed on from the face before (rhs.inl:1212-1214);
+   // that face is also the next cell's minus face.
+   template<int DIR>
+   __device__ __forceinline__ void stress(double *ct, const double *v0, double mu0, double hp, double hm) const
+   {
+      const Faces2 F = faces<DIR>();
+      const Transverse<DIR> G0 = transverse<DIR>(p.o, v0);
+      double Fp[4], Fm[4], v[3];
+      {
+         const uint32_t o = p.o + up[DIR];
 #pragma unroll
-      for (int i = 0; i < 3; i++) {
-         const double x = vel(p, i);
-         out[i] = (g0*(x - vel(pM1, i)) + g1*(vel(pP1, i) - x))*mm;
+         for (int i = 0; i < 3; i++) v[i] = vel(o, i);
+         const double mu = ldo<double, SOA>(f.mu, o);
+         const Transverse<DIR> G = transverse<DIR>(o, v);
+         Fp[3] = (stress_face<DIR>(Fp, F.wp, F.msp, v0, v, mu0, mu, F.own ? G : G0, G) - hp);
+         if (F.own) Fm[3] = (stress_face<DIR>(Fm, F.wp, F.msp, v0, v, mu0, mu, G0, G) - hm);
+#pragma unroll
+         for (int i = 0; i < 4; i++) HTR_PIN(Fp[i]);
       }
-   }
-
-   // face flux of cell p with the carried transverse gradients g[0] (left)
-   // and those of q = p + 1 formed here into g[1]; g[1] moves to g[0]
-   __device__ void flux(double *Flux, const P3 &p, double g1[2][3], double g2[2][3]) const
-   {
-      const P3 q = wplus(g, DIR, p, 1);
-      deriv3<D1>(q, g1[1]);
-      deriv3<D2>(q, g2[1]);
-      flux_at(Flux, p, q, g1, g2);
+      if (!F.own) {
+         const uint32_t o = p.o + dn[DIR];
 #pragma unroll
-      for (int i = 0; i < 3; i++) { g1[0][i] = g1[1][i]; g2[0][i] = g2[1][i]; }
-   }
-
-   // The cell values the species part of a face reads, loaded once per cell:
-   // a line walk hands the right cell's values on as the next face's left.
-   struct SpCell {
-      double X[NS], Di[NS], rY[NS];
-      double rho, T, lam, W;      // W: molar weight of the mixture from X
-   };
-   __device__ void sp_load(SpCell &c, const P3 &p) const
-   {
-#pragma unroll
-      for (int i = 0; i < NS; i++) {
-         c.X[i] = ld<double>(f.MolarFracs, p, i);
-         c.Di[i] = ld<double>(f.Di, p, i);
-         c.rY[i] = ld<double>(f.Conserved, p, i);
-      }
-      c.rho = ld<double>(f.rho, p);
-      c.T = ld<double>(f.temperature, p);
-      c.lam = ld<double>(f.lam, p);
-      c.W = MX::MolarWeightFromX(m, c.X);
-   }
-
-   // GetDiffusionFlux (rhs.inl:1140-1218) at the face between cells P and Q
-   // (node type t and staggered metric m_s of the left cell), species part:
-   // the species fluxes into Flux[0..NS-1] and the heat flux (conduction +
-   // species enthalpy transport) returned
-   __device__ double species_cells(double *Flux, int t, double m_s, const SpCell &P, const SpCell &Q) const
-   {
-      const double rho_s = interp2(t, P.rho, Q.rho);
-      const double iMixW_s = 1.0/interp2(t, P.W, Q.W);
-      const double T_s = interp2(t, P.T, Q.T);
-      double heatFlux = interp2(t, P.lam, Q.lam)*m_s*(P.T - Q.T);
-      double ViCorr = 0.0;
-      double hs[NS];
-      MX::SpeciesEnthalpies(m, hs, T_s);
-#pragma unroll
-      for (int i = 0; i < NS; i++) {
-         const double YiVi = interp2(t, P.Di[i], Q.Di[i])*m_s*(P.X[i] - Q.X[i])*MX::SpeciesW(m, i)*iMixW_s;
-         Flux[i] = -rho_s*YiVi;
-         heatFlux += rho_s*YiVi*hs[i];
-         ViCorr += YiVi;
+         for (int i = 0; i < 3; i++) v[i] = vel(o, i);
+         const double mu = ldo<double, SOA>(f.mu, o);
+         const Transverse<DIR> G = transverse<DIR>(o, v);
+         Fm[3] = (stress_face<DIR>(Fm, F.wm, F.msm, v, v0, mu, mu0, F.next ? G0 : G, G0) - hm);
       }
 #pragma unroll
-      for (int i = 0; i < NS; i++) {
-         const double corr = interp2(t, P.rY[i], Q.rY[i])*ViCorr;
-         Flux[i] += corr;
-         heatFlux -= corr*hs[i];
-      }
-      return heatFlux;
-   }
-
-   __device__ double species_at(double *Flux, const P3 &p, const P3 &q) const
-   {
-      SpCell P, Q;
-      sp_load(P, p);
-      sp_load(Q, q);
-      return species_cells(Flux, ld<int>(f.nType[DIR], p), ld<double>(f.m_s[DIR], p), P, Q);
-   }
-
-   // the cell values the momentum part of a face reads
-   struct StCell { double v[3], mu; };
-   __device__ void st_load(StCell &c, const P3 &p) const
-   {
-#pragma unroll
-      for (int i = 0; i < 3; i++) c.v[i] = vel(p, i);
-      c.mu = ld<double>(f.mu, p);
-   }
-
-   __device__ double stress_at(double *Flux, const P3 &p, const P3 &q, const double g1[2][3],
-                               const double g2[2][3]) const
-   {
-      StCell P, Q;
-      st_load(P, p);
-      st_load(Q, q);
-      return stress_cells(Flux, ld<int>(f.nType[DIR], p), ld<double>(f.m_s[DIR], p), P, Q, g1, g2);
-   }
-
-   // GetDiffusionFlux, momentum part: the viscous stress into Flux[0..2]
-   // and u.sigma returned (GetSigma, rhs.inl:1058-1137)
-   __device__ double stress_cells(double *Flux, int t, double m_s, const StCell &P, const StCell &Q,
-                                  const double g1[2][3], const double g2[2][3]) const
-   {
-      const double mu_s = interp2(t, P.mu, Q.mu);
-      const double *vp = P.v, *vq = Q.v;
-      double dn[3], s[3];
-#pragma unroll
-      for (int i = 0; i < 3; i++) dn[i] = m_s*(vq[i] - vp[i]);
-      if (DIR == 0) {
-         const double dUdY = interp2(t, g1[0][0], g1[1][0]);
-         const double dVdY = interp2(t, g1[0][1], g1[1][1]);
-         const double dUdZ = interp2(t, g2[0][0], g2[1][0]);
-         const double dWdZ = interp2(t, g2[0][2], g2[1][2]);
-         s[0] = mu_s*(4*dn[0] - 2*dVdY - 2*dWdZ)/3;
-         s[1] = mu_s*(dn[1] + dUdY);
-         s[2] = mu_s*(dn[2] + dUdZ);
-      } else if (DIR == 1) {
-         const double dUdX = interp2(t, g1[0][0], g1[1][0]);
-         const double dVdX = interp2(t, g1[0][1], g1[1][1]);
-         const double dVdZ = interp2(t, g2[0][1], g2[1][1]);
-         const double dWdZ = interp2(t, g2[0][2], g2[1][2]);
-         s[0] = mu_s*(dn[0] + dVdX);
-         s[1] = mu_s*(4*dn[1] - 2*dUdX - 2*dWdZ)/3;
-         s[2] = mu_s*(dn[2] + dVdZ);
-      } else {
-         const double dUdX = interp2(t, g1[0][0], g1[1][0]);
-         const double dWdX = interp2(t, g1[0][2], g1[1][2]);
-         const double dVdY = interp2(t, g2[0][1], g2[1][1]);
-         const double dWdY = interp2(t, g2[0][2], g2[1][2]);
-         s[0] = mu_s*(dn[0] + dWdX);
-         s[1] = mu_s*(dn[1] + dWdY);
-         s[2] = mu_s*(4*dn[2] - 2*dUdX - 2*dVdY)/3;
-      }
-
-#pragma unroll
-      for (int i = 0; i < 3; i++) Flux[i] = s[i];
-      double uSigma = 0.0;
-#pragma unroll
-      for (int i = 0; i < 3; i++) uSigma += interp2(t, vp[i], vq[i])*s[i];
-      return uSigma;
-   }
-
-   // GetDiffusionFlux (rhs.inl:1140-1218) at the face between p and q
-   __device__ void flux_at(double *Flux, const P3 &p, const P3 &q, const double g1[2][3], const double g2[2][3]) const
-   {
-      const double heatFlux = species_at(Flux, p, q);
-      const double uSigma = stress_at(Flux + NS, p, q, g1, g2);
-      Flux[NS+3] = (uSigma - heatFlux);
+      for (int i = 0; i < 4; i++) { ct[i] += (Fp[i] - Fm[i])*F.md; HTR_PIN(ct[i]); }
    }
 };
 
-// Faces walked along the line, divergence fused.  A thread takes one line
-// and one segment of L faces [j0, j0 + L) (a segment other than the first
-// also forms face j0 - 1), in the face order of the Euler passes: face j = 0
-// is the minus face of the line's first cell p0, at pm1 = p0 + offM1(nType);
-// face j >= 1 is the plus face of cell elo + j - 1.  The transverse velocity
-// gradients entering a face's left value are carried from the previous
-// face's right cell, as the reference does (rhs.inl:1212-1214): the face
-// cell itself, except for j = 1, where they belong to pm1 + 1 (different
-// from p0 only when offM1(nType[p0]) = 0, a staggered wall node).  Face j's
-// flux is differenced with face j-1's into Conserved_t of the cell between
-// them with m_d (rhs.inl:1264-1279).
-// The left cell's values of a face are the previous face's right cell's,
-// handed on in registers (reloaded at face 1, whose left cell p0 follows pm1
-// only when offM1(nType[p0]) = -1).
-// Two component groups, each walked by its own launch: G = 0 the species
-// fluxes, whose heat flux (conduction + species enthalpy transport) goes to
-// a face buffer H; G = 1 the viscous stress and the energy flux
-// u.sigma - H, read back per face.  Every value is the one the combined flux
-// forms; the split only halves the registers a thread holds.
-template<class MX, int G>
-struct DiffGroup {
-   static constexpr int LO = (G == 0) ? 0 : MX::NS;   // first conserved component
-   static constexpr int NC = (G == 0) ? MX::NS : 4;    // components of the group
-};
-
-template<class MX, int DIR, int G>
-__device__ __forceinline__ void diff_face(const Diffusion<MX, DIR> &D, double *Fc, const P3 &p, const P3 &q,
-                                          const double g1[2][3], const double g2[2][3], double *__restrict__ H,
-                                          uint32_t fid, bool owner)
+template<class MX, int DIRS, bool SOA>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4)))
+diffusion_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, uint32_t per)
 {
-   if constexpr (G == 0) {
-      const double heat = D.species_at(Fc, p, q);
-      if (owner) H[fid] = heat;
-   } else {
-      const double uSigma = D.stress_at(Fc, p, q, g1, g2);
-      Fc[3] = (uSigma - H[fid]);
+   constexpr int NS = MX::NS;
+   P3 p;
+   if (!strip_cell(g, per, p)) return;
+   const Diffusion<MX, DIRS, SOA> D(f, *mix, g, p);
+   // species first, then momentum and energy, so that the species' cell values
+   // are not held beside the velocity gradients; only the faces' heat fluxes
+   // pass from one to the other
+   double hp[3], hm[3];
+   {
+      DiffCell<MX, SOA> C0;
+      C0.load(f, *mix, p.o);
+      double ct[NS];
+#pragma unroll
+      for (int i = 0; i < NS; i++) ct[i] = ldo<double, SOA>(f.Conserved_t, p.o, i);
+      if constexpr ((DIRS & 4) != 0) D.template species<2>(ct, C0, hp[2], hm[2]);
+      if constexpr ((DIRS & 2) != 0) D.template species<1>(ct, C0, hp[1], hm[1]);
+      if constexpr ((DIRS & 1) != 0) D.template species<0>(ct, C0, hp[0], hm[0]);
+#pragma unroll
+      for (int i = 0; i < NS; i++) *ptr_o<double, SOA>(f.Conserved_t, p.o, i) = ct[i];
    }
+   double v0[3], ct[4];
+#pragma unroll
+   for (int i = 0; i < 3; i++) v0[i] = D.vel(p.o, i);
+   const double mu0 = ldo<double, SOA>(f.mu, p.o);
+#pragma unroll
+   for (int i = 0; i < 4; i++) ct[i] = ldo<double, SOA>(f.Conserved_t, p.o, NS + i);
+   if constexpr ((DIRS & 4) != 0) D.template stress<2>(ct, v0, mu0, hp[2], hm[2]);
+   if constexpr ((DIRS & 2) != 0) D.template stress<1>(ct, v0, mu0, hp[1], hm[1]);
+   if constexpr ((DIRS & 1) != 0) D.template stress<0>(ct, v0, mu0, hp[0], hm[0]);
+#pragma unroll
+   for (int i = 0; i < 4; i++) *ptr_o<double, SOA>(f.Conserved_t, p.o, NS + i) = ct[i];
 }
 
-template<class MX, int DIR, int G>
-__global__ void __launch_bounds__(256)
-diffusion_walk_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, double *__restrict__ H, int L,
-                      uint32_t nseg, uint32_t nunits)
-{
-   const uint32_t u = blockIdx.x*blockDim.x + threadIdx.x;
-   if (u >= nunits) return;
-   constexpr int A = Faces<DIR>::A, B = Faces<DIR>::B;
-   using K = DiffGroup<MX, G>;
-   uint32_t line, seg;
-   if (DIR == 0) { line = u/nseg; seg = u - line*nseg; }
-   else {
-      const uint32_t nl = (uint32_t)g.esz[A]*(uint32_t)g.esz[B];
-      seg = u/nl; line = u - seg*nl;
-   }
-   const int j0 = (int)seg*L;
-   const int j1 = min(j0 + L, g.esz[DIR] + 1);
-   int c[3];
-   c[A] = g.elo[A] + (int)(line % (uint32_t)g.esz[A]);
-   c[B] = g.elo[B] + (int)(line / (uint32_t)g.esz[A]);
-   c[DIR] = g.elo[DIR];
-   const P3 p0 = mkp(g, c[0], c[1], c[2]);
-   const P3 pm1 = wminus(g, DIR, p0, c_st.Cp[ld<int>(f.nType[DIR], p0)][1]);
-   int j = (j0 == 0) ? 0 : j0 - 1;
-   P3 cell = pm1, gl = pm1;
-   if (j > 0) {
-      cell = p0;
-      setc(g, cell, DIR, g.elo[DIR] + j - 1);
-      gl = (j == 1) ? wplus(g, DIR, pm1, 1) : cell;
-   }
-   using D_t = Diffusion<MX, DIR>;
-   D_t D{f, *mix, g};
-   double g1[2][3], g2[2][3], Fm[K::NC], Fc[K::NC];
-   // species group: the left cell's values, handed on from the previous
-   // face's right cell (reloaded at face 1, whose left cell p0 follows pm1
-   // only when offM1(nType[p0]) = -1)
-   using Cell = std::conditional_t<G == 0, typename D_t::SpCell, typename D_t::StCell>;
-   auto load = [&](Cell &c, const P3 &p) {
-      if constexpr (G == 0) D.sp_load(c, p); else D.st_load(c, p);
-   };
-   Cell P;
-   auto face = [&](const P3 &p, int jj, double *F) {
-      const P3 q = wplus(g, DIR, p, 1);
-      Cell Q;
-      load(Q, q);
-      const int t = ld<int>(f.nType[DIR], p);
-      const double m_s = ld<double>(f.m_s[DIR], p);
-      const uint32_t fid = Faces<DIR>::id(g, line, jj);
-      if constexpr (G == 0) {
-         const double heat = D.species_cells(F, t, m_s, P, Q);
-         if (jj >= j0) H[fid] = heat;
-      } else {
-         D.template deriv3<D_t::D1>(q, g1[1]);
-         D.template deriv3<D_t::D2>(q, g2[1]);
-         F[3] = (D.stress_cells(F, t, m_s, P, Q, g1, g2) - H[fid]);
-#pragma unroll
-         for (int i = 0; i < 3; i++) { g1[0][i] = g1[1][i]; g2[0][i] = g2[1][i]; }
-      }
-      P = Q;
-   };
-   load(P, cell);
-   if constexpr (G == 1) {
-      D.template deriv3<D_t::D1>(gl, g1[0]);
-      D.template deriv3<D_t::D2>(gl, g2[0]);
-   }
-   face(cell, j, Fm);
-   for (j++; j < j1; j++) {
-      cell = (j == 1) ? p0 : wplus(g, DIR, cell, 1);
-      if (j == 1) load(P, cell);
-      face(cell, j, Fc);
-      const double m = ld<double>(f.m_d[DIR], cell);
-#pragma unroll
-      for (int i = 0; i < K::NC; i++) {
-         at<double>(f.Conserved_t, cell, K::LO + i) += (Fc[i] - Fm[i])*m;
-         Fm[i] = Fc[i];
-      }
-   }
-}
-
-// x sweep: lanes on consecutive faces.  The faces of all rows are numbered
-// row-major (face j of row r is r (esz + 1) + j, its face id), and a wave
-// takes XD_OUT = 62 consecutive ones (lanes 2..63), so a wave may span the
-// end of one row and the start of the next: every lane forms the transverse
-// gradients of its right cell q, and takes those of its left cell and its
-// FluxM from lane l-1 (wave shuffles), so lanes 0 and 1 serve as the halo;
-// lane l-1 holds face j-1 of the same row whenever j >= 1, and face 0 takes
-// its left gradients at pm1 itself (rhs.inl:1253-1254) and adds no
-// divergence.
-constexpr int XD_OUT = 62;
-
-template<class MX, int G>
-__global__ void __launch_bounds__(256)
-diffusion_x_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, double *__restrict__ H,
-                   uint32_t nfx, uint32_t nwaves)
-{
-   using D_t = Diffusion<MX, 0>;
-   using K = DiffGroup<MX, G>;
-   const uint32_t wave = (blockIdx.x*blockDim.x + threadIdx.x) >> 6;
-   if (wave >= nwaves) return;                                      // whole waves
-   const int lane = threadIdx.x & 63;
-   const int esz = g.esz[0];
-   const int gf = (int)(wave*XD_OUT) + lane - 2;                    // face id of this lane
-   const bool live = gf >= 0 && (uint32_t)gf < nfx;
-   uint32_t row = 0;
-   int j = esz + 1;                                                  // (no face)
-   if (live) {
-      row = (uint32_t)gf/(uint32_t)(esz + 1);
-      j = gf - (int)(row*(uint32_t)(esz + 1));
-   }
-   const P3 prow = mkp(g, g.elo[0], g.elo[1] + (int)(row % (uint32_t)g.esz[1]),
-                       g.elo[2] + (int)(row/(uint32_t)g.esz[1]));
-   P3 p = wplus(g, 0, prow, j - 1);                                  // left cell of face j
-   if (j == 0) p = wminus(g, 0, prow, c_st.Cp[ld<int>(f.nType[0], prow)][1]);
-   const P3 q = wplus(g, 0, p, 1);
-   D_t D{f, *mix, g};
-   double g1[2][3], g2[2][3];
-   if constexpr (G == 1) {
-#pragma unroll
-      for (int i = 0; i < 3; i++) { g1[1][i] = 0.0; g2[1][i] = 0.0; }
-      if (live) {
-         D.template deriv3<D_t::D1>(q, g1[1]);
-         D.template deriv3<D_t::D2>(q, g2[1]);
-      }
-#pragma unroll
-      for (int i = 0; i < 3; i++) { g1[0][i] = __shfl_up(g1[1][i], 1, 64); g2[0][i] = __shfl_up(g2[1][i], 1, 64); }
-   }
-   double Fc[K::NC];
-#pragma unroll
-   for (int i = 0; i < K::NC; i++) Fc[i] = 0.0;
-   if (lane >= 1 && live && j >= 0) {
-      if constexpr (G == 1) {
-         if (j == 0) {
-            D.template deriv3<D_t::D1>(p, g1[0]);
-            D.template deriv3<D_t::D2>(p, g2[0]);
-         }
-      }
-      diff_face<MX, 0, G>(D, Fc, p, q, g1, g2, H, (uint32_t)gf, lane >= 2);
-   }
-   double Fm[K::NC];
-#pragma unroll
-   for (int i = 0; i < K::NC; i++) Fm[i] = __shfl_up(Fc[i], 1, 64);
-   if (lane >= 2 && live && j >= 1) {
-      const double m = ld<double>(f.m_d[0], p);
-#pragma unroll
-      for (int i = 0; i < K::NC; i++) at<double>(f.Conserved_t, p, K::LO + i) += (Fc[i] - Fm[i])*m;
-   }
-}
-
-template<class MX, int DIR>
+template<class MX, int DIRS>
 static int launch_diff(const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s)
 {
-   const int64_t ncells = exec_cells(g);
-   if (ncells == 0) return HTR_OK;
-   const int64_t nfaces = Faces<DIR>::count(g);
-   if (nfaces >= (1ll << 31)) return set_error(HTR_E_UNSUPPORTED, "diffusion: too many faces");
-   Workspace *wp = workspace(s);
-   if (!wp) return HTR_E_DEVICE;
-   int rc = workspace_faces(*wp, nfaces, 0, 0);
-   if (rc) return rc;
-   double *H = wp->faces;                          // heat flux per face
-   if constexpr (DIR == 0) {
-      // a lane's face id, below nwaves*XD_OUT + 62 <= nfaces + 123, stays an int
-      if (nfaces + 128 >= (1ll << 31)) return set_error(HTR_E_UNSUPPORTED, "diffusion: too many faces");
-      const int64_t nwaves = (nfaces + XD_OUT - 1)/XD_OUT;
-      HTR_LAUNCH("diffusion_species_x", (diffusion_x_kernel<MX, 0>), dim3(grid_for(nwaves*64, 256)), dim3(256), 0, s,
-                 f, mix, g, H, (uint32_t)nfaces, (uint32_t)nwaves);
-      if ((rc = check_launch("diffusion_x_kernel"))) return rc;
-      HTR_LAUNCH("diffusion_stress_x", (diffusion_x_kernel<MX, 1>), dim3(grid_for(nwaves*64, 256)), dim3(256), 0, s,
-                 f, mix, g, H, (uint32_t)nfaces, (uint32_t)nwaves);
-      return check_launch("diffusion_x_kernel");
+   if (exec_cells(g) == 0) return HTR_OK;
+   const StripGrid sg(g);
+   const char *name = (DIRS == 7) ? "diffusion" : (DIRS == 1) ? "diffusion_x" : (DIRS == 2) ? "diffusion_y" : "diffusion_z";
+   if (g.soa) {
+      HTR_LAUNCH(name, (diffusion_kernel<MX, DIRS, true>), dim3(sg.blocks), dim3(256), 0, s, f, mix, g, sg.per);
    } else {
-      const int L = walk_segment(DIR, (int64_t)g.esz[Faces<DIR>::A]*g.esz[Faces<DIR>::B], (int64_t)g.esz[DIR] + 1);
-      const int64_t nseg = ((int64_t)g.esz[DIR] + 1 + L - 1)/L;
-      const int64_t nunits = nseg*g.esz[Faces<DIR>::A]*g.esz[Faces<DIR>::B];
-      if (nunits >= (1ll << 31)) return set_error(HTR_E_UNSUPPORTED, "diffusion: too many line segments");
-      HTR_LAUNCH(HTR_DIR_NAME("diffusion_species", DIR), (diffusion_walk_kernel<MX, DIR, 0>),
-                 dim3(grid_for(nunits, 256)), dim3(256), 0, s, f, mix, g, H, L, (uint32_t)nseg, (uint32_t)nunits);
-      if ((rc = check_launch("diffusion_walk_kernel"))) return rc;
-      HTR_LAUNCH(HTR_DIR_NAME("diffusion_stress", DIR), (diffusion_walk_kernel<MX, DIR, 1>),
-                 dim3(grid_for(nunits, 256)), dim3(256), 0, s, f, mix, g, H, L, (uint32_t)nseg, (uint32_t)nunits);
-      return check_launch("diffusion_walk_kernel");
+      HTR_LAUNCH(name, (diffusion_kernel<MX, DIRS, false>), dim3(sg.blocks), dim3(256), 0, s, f, mix, g, sg.per);
    }
+   return check_launch("diffusion_kernel");
 }
 
+// dirs: one direction's bit, or 7 for all three (in the order z, y, x)
 template<class MX>
-int diffusion_dispatch(int dir, const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s)
+int diffusion_dispatch(int dirs, const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s)
 {
-   if (dir == 0) return launch_diff<MX, 0>(f, mix, g, s);
-   if (dir == 1) return launch_diff<MX, 1>(f, mix, g, s);
-   if (dir == 2) return launch_diff<MX, 2>(f, mix, g, s);
-   return set_error(HTR_E_ARG, "diffusion: bad direction %d", dir);
+   switch (dirs) {
+      case 1: return launch_diff<MX, 1>(f, mix, g, s);
+      case 2: return launch_diff<MX, 2>(f, mix, g, s);
+      case 4: return launch_diff<MX, 4>(f, mix, g, s);
+      case 7: return launch_diff<MX, 7>(f, mix, g, s);
+      default: return set_error(HTR_E_ARG, "diffusion: bad directions %d", dirs);
+   }
 }
 
 template int diffusion_dispatch<MixCP>(int, const htr_fields &, const DMix *, const Geo &, hipStream_t);

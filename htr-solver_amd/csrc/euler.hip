@@ -11,13 +11,13 @@
 // one (or of the first cell itself at a staggered left boundary).  Passes per
 // direction, all with consecutive lanes on x-adjacent cells:
 //   hybrid: classify faces (sensor) into a compacted TENO list; TENO faces in
-//     three passes (Roe record, characteristic components, back-projection
-//     and limiter) into a face buffer; then the KG walk: one thread per line
-//     segment carries the pair sums and FluxM along the sweep and
-//     differences the fluxes into Conserved_t, reading TENO faces back;
-//   pure TENO family: the three TENO passes over every face, then a
-//     divergence pass over the face buffer;
-//   pure KG: the KG walk alone.
+//     two passes (Roe record; characteristic components and back-projection)
+//     and the limiter into a face buffer; then the KG pass: one thread per
+//     cell forms both its faces and differences them into Conserved_t, reading
+//     TENO faces back (for all directions at once in a full right-hand side);
+//   pure TENO family: the TENO passes over every face, then a divergence pass
+//     over the face buffer;
+//   pure KG: the KG pass alone.
 // The TENO passes evaluate the characteristic projection one component at a
 // time (left-eigenvector rows of rhs.inl:436-505 with the per-point sums
 // hoisted), so no 6 x nEq split-flux arrays are held in registers.
@@ -520,328 +520,176 @@ euler_classify_kernel(const htr_fields f, const Geo g, int64_t nfaces, int32_t *
    }
 }
 
-// ---- Kennedy-Gruber faces walked along the line, divergence fused ----------
-// KGFluxReconstruction (rhs.inl:79-135) needs, at the face of cell p, the
-// pair sums S(p-m, p-m+l+1) for l < KOrder, m <= l: spans 1..3 with left
-// cells p-2..p.  Walking a line in face order, the pairs that start at p
-// (S(p,p+1), S(p,p+2), S(p,p+3)) are new at face p and the others were
-// formed at faces p-1 and p-2, which is the reference's ring buffer of pair
-// sums kept in registers.  The sums enter in the reference's order (l
-// outer, m inner).  The flux of face j is then differenced with that of
-// face j-1 into Conserved_t of the cell between them (rhs.inl:876-887), so
-// no KG face flux goes through memory; TENO faces of the hybrid scheme are
-// read from the face buffer the TENO passes wrote.
+// ---- Kennedy-Gruber faces of a cell, divergence fused ------------------------
+// KGFluxReconstruction (rhs.inl:79-135) of the face on the plus side of cell p
+// is the sum over spans l+1 = 1..3 and shifts m <= l of the pair sums
+// S(p-m, p-m+l+1), l outer, m inner.  A thread forms both faces of its cell
+// along every direction of the launch from the seven cells p-3..p+3 of the
+// line, in the reference's order (nine distinct pairs serve the two faces),
+// and adds (F+ - F-) m_e to Conserved_t, which it reads and writes once for
+// all directions; TENO faces of the hybrid scheme come from the face buffers
+// the TENO passes wrote.
 //
-// The conserved components are split in two groups, each walked by its own
-// wave: G = 0 the species (pair values rho Y_i), G = 1 momentum, energy and
-// the pressure sum.  A thread takes one line and one segment of L faces
-// [j0, j0 + L); a segment other than the first also forms face j0 - 1.
-template<class MX, int G>
-struct KGGroup {
-   static constexpr int NS = MX::NS;
-   static constexpr int LO = (G == 0) ? 0 : NS;       // first conserved component of the group
-   static constexpr int NC = (G == 0) ? NS : 4;       // conserved components of the group
-   static constexpr int NP = (G == 0) ? NS : 5;       // pair values (G = 1: + pressure sum)
-};
+// Forming every face twice costs 1000 FP64 operations per cell instead of
+// 500, which is little beside what it removes.  The walks along the lines
+// that this replaces (a pass per direction and component group, the ring of
+// pair sums carried in registers) read and wrote Conserved_t three times and
+// the stencil fields six times, and each thread took the faces of its segment
+// one after another, node type -> table -> sensor -> flux -> Conserved_t, as
+// a chain of dependent loads: they waited 88 % of their cycles.  Here the
+// loads of a component are independent of each other, no thread waits for
+// another, and a small box has a thread per cell instead of one per eight.
+// Bound by the number of loads: a 64-lane 8-byte load takes the CU's address
+// unit 16 cycles (measured, from L1, contiguous or not), 230 of them per cell.
+// All three directions, measured with the walks in brackets: 256^3 air 3.9
+// (5.0) ms, 512x256x128 boundary layer 2.9 (4.6) ms, 32^3 one species 15 (155)
+// us; one direction of 256^3 air without TENO faces 1.2 (1.66) ms.
+struct KGFaces { const double *f[3]; };      // face buffers of the directions' TENO faces
 
-template<class MX, int DIR, int G>
-struct KGCell {
-   using K = KGGroup<MX, G>;
-   double rho, un, v[K::NP];
-   __device__ void load(const htr_fields &f, const htr_view &hv, const P3 &p)
-   {
-      rho = ld<double>(f.rho, p);
-      un = ld<double>(f.velocity, p, DIR);
-      if constexpr (G == 0) {
-#pragma unroll
-         for (int i = 0; i < K::NS; i++) v[i] = ld<double>(f.MassFracs, p, i);
-      } else {
-#pragma unroll
-         for (int i = 0; i < 3; i++) v[i] = ld<double>(f.velocity, p, i);
-         v[3] = ld<double>(hv, p);
-         v[4] = ld<double>(f.pressure, p);
-      }
-   }
-};
-
-// pair sum S(a, b) of the group (rhs.inl:42-75)
-template<class MX, int DIR, int G>
-__device__ __forceinline__ void kg_pair(double *S, const KGCell<MX, DIR, G> &a, const KGCell<MX, DIR, G> &b)
+// hybrid sensor of a face (rhs.inl:818-820) from the sensors of the cells
+// before, at and after its left cell, whose node type is t: the stencil
+// offsets of a node type are 0 or the natural ones
+__device__ __forceinline__ bool face_is_kg(int t, bool sm, bool s0, bool sp)
 {
-   using K = KGGroup<MX, G>;
-   const double rhom = a.rho + b.rho;
-   const double vm = -(a.un + b.un);
-#pragma unroll
-   for (int i = 0; i < K::NC; i++) S[i] = rhom*vm*(a.v[i] + b.v[i]);
-   if constexpr (G == 1) S[4] = a.v[4] + b.v[4];
+   return (t == L_S_node || t == L_C_node || sm) && s0 && (t == R_S_node || t == R_C_node || sp);
 }
 
-template<class MX, int DIR, int G>
-struct KGRing {
-   using K = KGGroup<MX, G>;
-   using Cell = KGCell<MX, DIR, G>;
-   double R2[K::NP], R3a[K::NP], R3b[K::NP];   // S(p-1,p+1), S(p-1,p+2), S(p-2,p+1) at face p
-
-   __device__ void warm(const htr_fields &f, const htr_view &hv, const Geo &g, const P3 &p)
-   {
-      Cell a, b;
-      a.load(f, hv, wminus(g, DIR, p, -1));
-      b.load(f, hv, wplus(g, DIR, p, 1));
-      kg_pair<MX, DIR, G>(R2, a, b);
-      b.load(f, hv, wplus(g, DIR, p, 2));
-      kg_pair<MX, DIR, G>(R3a, a, b);
-      a.load(f, hv, wminus(g, DIR, p, -2));
-      b.load(f, hv, wplus(g, DIR, p, 1));
-      kg_pair<MX, DIR, G>(R3b, a, b);
-   }
-
-   // face of cell p (node type t): KG flux of the group into Flux when kg,
-   // and the ring advanced to face p+1 in any case
-   __device__ void step(const htr_fields &f, const htr_view &hv, const Geo &g, const P3 &p, int t, bool kg,
-                        double *Flux)
-   {
-      Cell a, b;
-      a.load(f, hv, p);
-      double fl[K::NP], N[K::NP];
-      const int order = c_st.KOrder[t];
-      b.load(f, hv, wplus(g, DIR, p, 1));
-      kg_pair<MX, DIR, G>(N, a, b);                                   // l = 0: S(p,p+1)
-      {
-         const double c = c_st.KCoeff[t][0];
-#pragma unroll
-         for (int i = 0; i < K::NP; i++) fl[i] = (order > 0) ? c*N[i] : 0.0;
-      }
-      b.load(f, hv, wplus(g, DIR, p, 2));
-      kg_pair<MX, DIR, G>(N, a, b);                                   // l = 1: S(p,p+2) + S(p-1,p+1)
-      if (order > 1) {
-         const double c = c_st.KCoeff[t][1];
-#pragma unroll
-         for (int i = 0; i < K::NP; i++) fl[i] += c*(N[i] + R2[i]);
-      }
-#pragma unroll
-      for (int i = 0; i < K::NP; i++) R2[i] = N[i];
-      b.load(f, hv, wplus(g, DIR, p, 3));
-      kg_pair<MX, DIR, G>(N, a, b);                                   // l = 2: S(p,p+3) + S(p-1,p+2) + S(p-2,p+1)
-      if (order > 2) {
-         const double c = c_st.KCoeff[t][2];
-#pragma unroll
-         for (int i = 0; i < K::NP; i++) fl[i] += c*((N[i] + R3a[i]) + R3b[i]);
-      }
-#pragma unroll
-      for (int i = 0; i < K::NP; i++) { R3b[i] = R3a[i]; R3a[i] = N[i]; }
-      if (!kg) return;
-      if (t == L_S_node || t == Rm1_S_node) {
-         // staggered-node flux (rhs.inl:92-110)
-         const P3 q = (t == L_S_node) ? p : wplus(g, DIR, p, c_st.Cp[t][2]);
-         const double u = ld<double>(f.velocity, q, DIR);
-#pragma unroll
-         for (int i = 0; i < K::NC; i++) Flux[i] = -(ld<double>(f.Conserved, q, K::LO + i)*u);
-         if constexpr (G == 1) {
-            const double pr = ld<double>(f.pressure, q);
-            Flux[DIR] -= pr;
-            Flux[3] -= pr*u;
-         }
-         return;
-      }
-#pragma unroll
-      for (int i = 0; i < K::NC; i++) Flux[i] = 0.25*fl[i];
-      if constexpr (G == 1) Flux[DIR] -= fl[4];
-   }
-};
-
-template<class MX, int DIR, bool ALL_KG, int G>
-__device__ void kg_walk(const htr_fields &f, const Geo &g, const htr_view &hv, const double *__restrict__ F,
-                        int64_t nfaces, uint32_t line, int j0, int j1, const htr_view &dec)
+template<class MX, int DIR, bool ALL_KG, bool SOA>
+__device__ __forceinline__ void kg_dir(const htr_fields &f, const Geo &g, const htr_view &hv,
+                                       const double *__restrict__ F, const P3 &p, double *ct, const htr_view &dec)
 {
-   using K = KGGroup<MX, G>;
-   constexpr int A = Faces<DIR>::A, B = Faces<DIR>::B;
-   int c[3];
-   c[A] = g.elo[A] + (int)(line % (uint32_t)g.esz[A]);
-   c[B] = g.elo[B] + (int)(line / (uint32_t)g.esz[A]);
-   c[DIR] = g.elo[DIR];
-   const P3 p0 = mkp(g, c[0], c[1], c[2]);
-   KGRing<MX, DIR, G> ring;
-   double Fm[K::NC], Fc[K::NC];
-   auto face = [&](const P3 &p, int t, int j, double *Fl) {
-      const bool kg = ALL_KG || hybrid_kg<DIR>(f, g, p, t);
-      ring.step(f, hv, g, p, t, kg, Fl);
-      if (!kg) {
-         const uint32_t fid = Faces<DIR>::id(g, line, j);
+   constexpr int NS = MX::NS, NEQ = MX::NEQ;
+   constexpr int Z = 3;                              // index of the cell itself
+   uint32_t o[7];
+   {
+      int c = p.c[DIR];
+      o[Z] = p.o;
 #pragma unroll
-         for (int i = 0; i < K::NC; i++) Fl[i] = face_ld<MX::NEQ>(F, fid, K::LO + i);
-      } else if (G == 0 && dec.ptr) {
-         at<uint32_t>(dec, p) = 1;
+      for (int k = 1; k <= 3; k++) { o[Z+k] = o[Z+k-1]; step_up(g, DIR, c, o[Z+k]); }
+      c = p.c[DIR];
+#pragma unroll
+      for (int k = 1; k <= 3; k++) { o[Z-k] = o[Z-k+1]; step_down(g, DIR, c, o[Z-k]); }
+   }
+   const int t = ldo<int, SOA>(f.nType[DIR], o[Z]), tm = ldo<int, SOA>(f.nType[DIR], o[Z-1]);
+   const double m = ldo<double, SOA>(f.m_e[DIR], o[Z]);
+   // the minus face of a line's first cell is the face of p + offM1(nType)
+   // (rhs.inl:800-817): the previous cell's, but the cell's own at a left
+   // boundary node
+   const bool first = p.c[DIR] == g.elo[DIR];
+   const bool own = first && (t == L_S_node || t == L_C_node);
+   bool kgp = true, kgm = true;
+   if constexpr (!ALL_KG) {
+      const bool s2 = ldo<uint8_t, SOA>(f.shockSensor[DIR], o[Z-2]), s1 = ldo<uint8_t, SOA>(f.shockSensor[DIR], o[Z-1]),
+                 s0 = ldo<uint8_t, SOA>(f.shockSensor[DIR], o[Z]), sp = ldo<uint8_t, SOA>(f.shockSensor[DIR], o[Z+1]);
+      kgp = face_is_kg(t, s1, s0, sp);
+      kgm = own ? kgp : face_is_kg(tm, s2, s1, s0);
+   }
+   if (dec.ptr) {
+      if (kgp) *ptr_o<uint32_t, SOA>(dec, o[Z]) = 1;
+      if (first && kgm) *ptr_o<uint32_t, SOA>(dec, own ? o[Z] : o[Z-1]) = 1;
+   }
+   // span sums of a face: sixth order inside, a boundary node type has fewer
+   // spans and the coefficients of that order
+   const bool std = wave_all(t == Std_node && tm == Std_node);
+   int op = 3, om = 3;
+   if (!std) { op = c_st.KOrder[t]; om = c_st.KOrder[tm]; }
+   auto spans = [&](int order, double a, double b, double c) {
+      if (std) {
+         double l = (3.0/4.0)*a;
+         l += (-3.0/20.0)*b;
+         l += (1.0/60.0)*c;
+         return l;
+      }
+      double l = (order > 0) ? (order > 2 ? 3.0/4.0 : order > 1 ? 2.0/3.0 : 0.5)*a : 0.0;
+      if (order > 1) l += (order > 2 ? -3.0/20.0 : -1.0/12.0)*b;
+      if (order > 2) l += (1.0/60.0)*c;
+      return l;
+   };
+   // faces whose flux is not the split form's: TENO faces, from the face
+   // buffer, and those of staggered nodes (rhs.inl:92-110), from the cell they
+   // lie on
+   const bool sgp = kgp && (t == L_S_node || t == Rm1_S_node), sgm = kgm && (tm == L_S_node || tm == Rm1_S_node);
+   const bool others = !wave_all(kgp && kgm && !sgp && !sgm);
+   uint32_t fid = 0;
+   if constexpr (!ALL_KG) {
+      constexpr int A = Faces<DIR>::A, B = Faces<DIR>::B;
+      const uint32_t line = (uint32_t)(p.c[A] - g.elo[A]) + (uint32_t)(p.c[B] - g.elo[B])*(uint32_t)g.esz[A];
+      fid = Faces<DIR>::id(g, line, p.c[DIR] - g.elo[DIR] + 1);
+   }
+   auto take = [&](bool kg, bool stag, uint32_t id, uint32_t q, int i, double &fl) {
+      if (!kg) {
+         fl = face_ld<NEQ>(F, id, i);
+      } else if (stag) {
+         const double u = ldo<double, SOA>(f.velocity, q, DIR);
+         fl = -(ldo<double, SOA>(f.Conserved, q, i)*u);
+         if (i == NS + DIR) fl -= ldo<double, SOA>(f.pressure, q);
+         if (i == NS + 3) fl -= ldo<double, SOA>(f.pressure, q)*u;
       }
    };
-   int j;
+   // (rho_a + rho_b)(-(u_a + u_b)) of the pairs: plus face (0,1) (0,2) (-1,1)
+   // (0,3) (-1,2) (-2,1), minus face (-1,0) (-1,1) (-2,0) (-1,2) (-2,1) (-3,0)
+   double rv[9];
+   {
+      double r[7], u[7];
+#pragma unroll
+      for (int k = 0; k < 7; k++) { r[k] = ldo<double, SOA>(f.rho, o[k]); u[k] = ldo<double, SOA>(f.velocity, o[k], DIR); }
+      auto prod = [&](int a, int b) { return (r[Z+a] + r[Z+b])*(-(u[Z+a] + u[Z+b])); };
+      rv[0] = prod(0, 1);  rv[1] = prod(0, 2);  rv[2] = prod(-1, 1);
+      rv[3] = prod(0, 3);  rv[4] = prod(-1, 2); rv[5] = prod(-2, 1);
+      rv[6] = prod(-1, 0); rv[7] = prod(-2, 0); rv[8] = prod(-3, 0);
+   }
+   // the two faces' span sums of one component: S(a, b) = rv(a, b) (v_a + v_b),
+   // or v_a + v_b alone for the pressure
+   auto faces = [&](const double *v, bool weighted, double &lp, double &lm) {
+      auto S = [&](int k, int a, int b) { const double s = v[Z+a] + v[Z+b]; return weighted ? rv[k]*s : s; };
+      const double p1 = S(0, 0, 1), p2 = S(1, 0, 2), q = S(2, -1, 1), p3 = S(3, 0, 3), a4 = S(4, -1, 2), a5 = S(5, -2, 1);
+      const double m1 = S(6, -1, 0), m2 = S(7, -2, 0), m3 = S(8, -3, 0);
+      lp = spans(op, p1, p2 + q, (p3 + a4) + a5);
+      lm = spans(om, m1, q + m2, (a4 + a5) + m3);
+   };
+#pragma unroll
+   for (int i = 0; i < NEQ; i++) {
+      double v[7], lp, lm;
+#pragma unroll
+      for (int k = 0; k < 7; k++)
+         v[k] = (i < NS) ? ldo<double, SOA>(f.MassFracs, o[k], i)
+              : (i < NS + 3) ? ldo<double, SOA>(f.velocity, o[k], i - NS) : ldo<double, SOA>(hv, o[k]);
+      faces(v, true, lp, lm);
+      double gp = 0.25*lp, gm = 0.25*lm;
+      if (i == NS + DIR) {
+#pragma unroll
+         for (int k = 0; k < 7; k++) v[k] = ldo<double, SOA>(f.pressure, o[k]);
+         faces(v, false, lp, lm);
+         gp -= lp;
+         gm -= lm;
+      }
+      if (others) {
+         take(kgp, sgp, fid, t == L_S_node ? o[Z] : o[Z+1], i, gp);
+         take(kgm, sgm, fid - Faces<DIR>::id(g, 0, 1), tm == L_S_node ? o[Z-1] : o[Z], i, gm);
+      }
+      if (own) gm = gp;
+      ct[i] += (gp - gm)*m;
+      // the sums are formed here, component by component: left to itself the
+      // compiler issues the loads of all components and directions first and
+      // holds 220 registers
+      HTR_PIN(ct[i]);
+   }
+}
+
+template<class MX, int DIRS, bool ALL_KG, bool SOA>
+__global__ void __launch_bounds__(256)
+euler_kg_kernel(const htr_fields f, const Geo g, const htr_view hv, const KGFaces F, uint32_t per, htr_view dec)
+{
    P3 p;
-   if (j0 == 0) {
-      // face 0 at p0 + offM1(nType[p0]) (rhs.inl:800-817)
-      const P3 q = wminus(g, DIR, p0, c_st.Cp[ld<int>(f.nType[DIR], p0)][1]);
-      ring.warm(f, hv, g, q);
-      face(q, ld<int>(f.nType[DIR], q), 0, Fm);
-      j = 1;
-      p = p0;
-   } else {
-      j = j0 - 1;
-      p = wplus(g, DIR, p0, j - 1);
-   }
-   ring.warm(f, hv, g, p);
-   if (j0 > 0) {
-      face(p, ld<int>(f.nType[DIR], p), j, Fm);
-      j++;
-      p = wplus(g, DIR, p, 1);
-   }
-   for (; j < j1; j++) {
-      face(p, ld<int>(f.nType[DIR], p), j, Fc);
-      const double m = ld<double>(f.m_e[DIR], p);
+   if (!strip_cell(g, per, p)) return;
+   double ct[MX::NEQ];
 #pragma unroll
-      for (int i = 0; i < K::NC; i++) {
-         at<double>(f.Conserved_t, p, K::LO + i) += (Fc[i] - Fm[i])*m;
-         Fm[i] = Fc[i];
-      }
-      p = wplus(g, DIR, p, 1);
-   }
-}
-
-// Work units: (line, segment) pairs, nseg segments of L faces per line; for
-// the x sweep consecutive units are consecutive segments of a line, for y
-// and z consecutive lines (x-adjacent cells).  One launch per component
-// group G.
-template<class MX, int DIR, bool ALL_KG, int G>
-__global__ void __launch_bounds__(256)
-euler_kg_walk_kernel(const htr_fields f, const Geo g, const htr_view hv, const double *__restrict__ F,
-                     int64_t nfaces, int L, uint32_t nseg, uint32_t nunits, htr_view dec)
-{
-   const uint32_t u = blockIdx.x*blockDim.x + threadIdx.x;
-   if (u >= nunits) return;
-   uint32_t line, seg;
-   if (DIR == 0) { line = u/nseg; seg = u - line*nseg; }
-   else {
-      const uint32_t nl = (uint32_t)g.esz[Faces<DIR>::A]*(uint32_t)g.esz[Faces<DIR>::B];
-      seg = u/nl; line = u - seg*nl;
-   }
-   const int j0 = (int)seg*L;
-   const int j1 = min(j0 + L, g.esz[DIR] + 1);
-   kg_walk<MX, DIR, ALL_KG, G>(f, g, hv, F, nfaces, line, j0, j1, dec);
-}
-
-// x sweep: lanes on consecutive faces.  Each row has esz + 4 slots, faces
-// j = -3 .. esz (the three before face 0 only form pairs), numbered
-// row-major across rows, and a wave takes XK_OUT = 61 consecutive slots
-// (lanes 3..63), so a wave may span the end of one row and the start of the
-// next.  Every lane forms the new pairs S(p,p+d) of its cell; a lane's older
-// pairs are those of lanes l-1 and l-2 and its FluxM is the flux of lane
-// l-1 (wave shuffles), so lanes 0..2 serve as the halo of lane 3; for a face
-// j >= 0 those lanes hold slots j-1 and j-2 of the same row.
-constexpr int XK_OUT = 61;
-
-template<class MX, bool ALL_KG, int G>
-__global__ void __launch_bounds__(256)
-euler_kg_x_kernel(const htr_fields f, const Geo g, const htr_view hv, const double *__restrict__ F,
-                  uint32_t nslot, uint32_t nwaves, htr_view dec)
-{
-   using K = KGGroup<MX, G>;
-   using Cell = KGCell<MX, 0, G>;
-   const uint32_t wave = (blockIdx.x*blockDim.x + threadIdx.x) >> 6;
-   if (wave >= nwaves) return;                                      // whole waves
-   const int lane = threadIdx.x & 63;
-   const int esz = g.esz[0];
-   const int gs = (int)(wave*XK_OUT) + lane - 3;                    // slot of this lane
-   const bool live = gs >= 0 && (uint32_t)gs < nslot;
-   uint32_t row = 0;
-   int j = esz + 1;                                                  // (no face)
-   if (live) {
-      row = (uint32_t)gs/(uint32_t)(esz + 4);
-      j = gs - (int)(row*(uint32_t)(esz + 4)) - 3;                    // face of this lane
-   }
-   const P3 prow = mkp(g, g.elo[0], g.elo[1] + (int)(row % (uint32_t)g.esz[1]),
-                       g.elo[2] + (int)(row/(uint32_t)g.esz[1]));
-   const P3 p = wplus(g, 0, prow, j - 1);                            // left cell of face j
-   double N1[K::NP], N2[K::NP], N3[K::NP];
-   int t = 0;
-   if (live) {
-      Cell a, b;
-      a.load(f, hv, p);
-      t = ld<int>(f.nType[0], p);
-      b.load(f, hv, wplus(g, 0, p, 1));
-      kg_pair<MX, 0, G>(N1, a, b);
-      b.load(f, hv, wplus(g, 0, p, 2));
-      kg_pair<MX, 0, G>(N2, a, b);
-      b.load(f, hv, wplus(g, 0, p, 3));
-      kg_pair<MX, 0, G>(N3, a, b);
-   } else {
+   for (int i = 0; i < MX::NEQ; i++) ct[i] = ldo<double, SOA>(f.Conserved_t, p.o, i);
+   if constexpr ((DIRS & 4) != 0) kg_dir<MX, 2, ALL_KG, SOA>(f, g, hv, F.f[2], p, ct, dec);
+   if constexpr ((DIRS & 2) != 0) kg_dir<MX, 1, ALL_KG, SOA>(f, g, hv, F.f[1], p, ct, dec);
+   if constexpr ((DIRS & 1) != 0) kg_dir<MX, 0, ALL_KG, SOA>(f, g, hv, F.f[0], p, ct, dec);
 #pragma unroll
-      for (int i = 0; i < K::NP; i++) { N1[i] = 0.0; N2[i] = 0.0; N3[i] = 0.0; }
-   }
-   double R2[K::NP], R3a[K::NP], R3b[K::NP];
-#pragma unroll
-   for (int i = 0; i < K::NP; i++) {
-      R2[i] = __shfl_up(N2[i], 1, 64);
-      R3a[i] = __shfl_up(N3[i], 1, 64);
-      R3b[i] = __shfl_up(N3[i], 2, 64);
-   }
-   double Fc[K::NC];
-#pragma unroll
-   for (int i = 0; i < K::NC; i++) Fc[i] = 0.0;
-   bool kg = false;
-   P3 q = p;                                                          // the face's cell
-   if (lane >= 2 && j >= 0 && live) {
-      int tq = t;
-      if (j == 0) {
-         // face 0 at p0 + offM1(nType[p0]) (rhs.inl:800-817): the natural
-         // left cell except at a staggered left boundary
-         const P3 p0 = wplus(g, 0, p, 1);
-         q = wminus(g, 0, p0, c_st.Cp[ld<int>(f.nType[0], p0)][1]);
-         tq = ld<int>(f.nType[0], q);
-      }
-      kg = ALL_KG || hybrid_kg<0>(f, g, q, tq);
-      if (!kg) {
-         const uint32_t fid = row*(uint32_t)(esz + 1) + (uint32_t)j;
-#pragma unroll
-         for (int i = 0; i < K::NC; i++) Fc[i] = face_ld<MX::NEQ>(F, fid, K::LO + i);
-      } else if (q.o != p.o) {
-         KGRing<MX, 0, G> ring;
-         ring.warm(f, hv, g, q);
-         ring.step(f, hv, g, q, tq, true, Fc);
-      } else if (t == L_S_node || t == Rm1_S_node) {
-         const P3 qs = (t == L_S_node) ? p : wplus(g, 0, p, c_st.Cp[t][2]);
-         const double u = ld<double>(f.velocity, qs, 0);
-#pragma unroll
-         for (int i = 0; i < K::NC; i++) Fc[i] = -(ld<double>(f.Conserved, qs, K::LO + i)*u);
-         if constexpr (G == 1) {
-            const double pr = ld<double>(f.pressure, qs);
-            Fc[0] -= pr;
-            Fc[3] -= pr*u;
-         }
-      } else {
-         // KGFluxReconstruction (rhs.inl:79-135), l outer, m inner
-         const int order = c_st.KOrder[t];
-         double fl[K::NP];
-         const double c0 = c_st.KCoeff[t][0], c1 = c_st.KCoeff[t][1], c2 = c_st.KCoeff[t][2];
-#pragma unroll
-         for (int i = 0; i < K::NP; i++) {
-            double v = (order > 0) ? c0*N1[i] : 0.0;
-            if (order > 1) v += c1*(N2[i] + R2[i]);
-            if (order > 2) v += c2*((N3[i] + R3a[i]) + R3b[i]);
-            fl[i] = v;
-         }
-#pragma unroll
-         for (int i = 0; i < K::NC; i++) Fc[i] = 0.25*fl[i];
-         if constexpr (G == 1) Fc[0] -= fl[4];
-      }
-   }
-   double Fm[K::NC];
-#pragma unroll
-   for (int i = 0; i < K::NC; i++) Fm[i] = __shfl_up(Fc[i], 1, 64);
-   if (lane >= 3 && live && j >= 0) {
-      if (G == 0 && kg && dec.ptr) at<uint32_t>(dec, q) = 1;
-      if (j >= 1) {
-         const double m = ld<double>(f.m_e[0], p);
-#pragma unroll
-         for (int i = 0; i < K::NC; i++) at<double>(f.Conserved_t, p, K::LO + i) += (Fc[i] - Fm[i])*m;
-      }
-   }
+   for (int i = 0; i < MX::NEQ; i++) *ptr_o<double, SOA>(f.Conserved_t, p.o, i) = ct[i];
 }
 
 // Pass 2: TENO-family faces, either all faces or the compacted list, in
@@ -1193,39 +1041,21 @@ static int teno_faces(const htr_fields &f, const DMix *mix, const Geo &g, const 
    return launch_teno<MX, DIR, HTR_EULER_TENO, true>(f, mix, g, hv, RK0, RK1, dt, w, nfaces, F, dec, s);
 }
 
-// The KG faces and the fused divergence of a hybrid (or pure KG, ALL) sweep
-// along DIR, the listed TENO faces read back from F
-template<class MX, int DIR, bool ALL>
-static int kg_walks(const htr_fields &f, const Geo &g, const htr_view &hv, const double *F, int64_t nfaces,
-                    const htr_view &dec, hipStream_t s)
+// The KG faces and the fused divergence of the sweeps DIRS (bit d: direction
+// d) of a hybrid (or pure KG, ALL) scheme, in the order z, y, x; the listed TENO
+// faces are read back from F
+template<class MX, int DIRS, bool ALL>
+static int kg_cells(const htr_fields &f, const Geo &g, const htr_view &hv, const KGFaces &F, const htr_view &dec,
+                    hipStream_t s)
 {
-   int rc;
-   if constexpr (DIR == 0) {
-      // esz + 4 slots per row; a lane's slot, below nwaves*XK_OUT + 61 <=
-      // nslot + 121, stays an int
-      const int64_t nslot = ((int64_t)g.esz[0] + 4)*g.esz[1]*g.esz[2];
-      if (nslot + 128 >= (1ll << 31)) return set_error(HTR_E_UNSUPPORTED, "euler: too many rows");
-      const int64_t nwaves = (nslot + XK_OUT - 1)/XK_OUT;
-      HTR_LAUNCH("euler_kg_species_x", (euler_kg_x_kernel<MX, ALL, 0>), dim3(grid_for(nwaves*64, 256)), dim3(256), 0,
-                 s, f, g, hv, F, (uint32_t)nslot, (uint32_t)nwaves, dec);
-      if ((rc = check_launch("euler_kg_x_kernel"))) return rc;
-      HTR_LAUNCH("euler_kg_flow_x", (euler_kg_x_kernel<MX, ALL, 1>), dim3(grid_for(nwaves*64, 256)), dim3(256), 0,
-                 s, f, g, hv, F, (uint32_t)nslot, (uint32_t)nwaves, dec);
-      return check_launch("euler_kg_x_kernel");
+   const StripGrid sg(g);
+   const char *name = (DIRS == 7) ? "euler_kg" : (DIRS == 1) ? "euler_kg_x" : (DIRS == 2) ? "euler_kg_y" : "euler_kg_z";
+   if (g.soa) {
+      HTR_LAUNCH(name, (euler_kg_kernel<MX, DIRS, ALL, true>), dim3(sg.blocks), dim3(256), 0, s, f, g, hv, F, sg.per, dec);
    } else {
-      const int L = walk_segment(DIR, (int64_t)g.esz[Faces<DIR>::A]*g.esz[Faces<DIR>::B], (int64_t)g.esz[DIR] + 1);
-      const int64_t nseg = ((int64_t)g.esz[DIR] + 1 + L - 1)/L;
-      const int64_t nunits = nseg*g.esz[Faces<DIR>::A]*g.esz[Faces<DIR>::B];
-      if (nunits >= (1ll << 31)) return set_error(HTR_E_UNSUPPORTED, "euler: too many line segments");
-      HTR_LAUNCH(HTR_DIR_NAME("euler_kg_species", DIR), (euler_kg_walk_kernel<MX, DIR, ALL, 0>),
-                 dim3(grid_for(nunits, 256)), dim3(256), 0, s, f, g, hv, F, nfaces, L, (uint32_t)nseg,
-                 (uint32_t)nunits, dec);
-      if ((rc = check_launch("euler_kg_walk_kernel"))) return rc;
-      HTR_LAUNCH(HTR_DIR_NAME("euler_kg_flow", DIR), (euler_kg_walk_kernel<MX, DIR, ALL, 1>),
-                 dim3(grid_for(nunits, 256)), dim3(256), 0, s, f, g, hv, F, nfaces, L, (uint32_t)nseg,
-                 (uint32_t)nunits, dec);
-      return check_launch("euler_kg_walk_kernel");
+      HTR_LAUNCH(name, (euler_kg_kernel<MX, DIRS, ALL, false>), dim3(sg.blocks), dim3(256), 0, s, f, g, hv, F, sg.per, dec);
    }
+   return check_launch("euler_kg_kernel");
 }
 
 // the caller's total-enthalpy array (workspace of stream s) as a view
@@ -1270,7 +1100,9 @@ static int launch_dir(const htr_fields &f, const DMix *mix, const Geo &g, double
       if ((rc = teno_faces<MX, DIR>(f, mix, g, hv, RK0, RK1, dt, w, nfaces, w.faces, dec, s))) return rc;
    }
    if constexpr (SCHEME == HTR_EULER_HYBRID || SCHEME == HTR_EULER_KG) {
-      return kg_walks<MX, DIR, SCHEME == HTR_EULER_KG>(f, g, hv, w.faces, nfaces, dec, s);
+      KGFaces F = {};
+      F.f[DIR] = w.faces;
+      return kg_cells<MX, 1 << DIR, SCHEME == HTR_EULER_KG>(f, g, hv, F, dec, s);
    } else {
       if ((rc = launch_teno<MX, DIR, SCHEME, false>(f, mix, g, hv, RK0, RK1, dt, w, nfaces, w.faces, dec, s))) return rc;
       HTR_LAUNCH(HTR_DIR_NAME("euler_divergence", DIR), (face_divergence_kernel<MX::NEQ, DIR>), dim3(grid_for(ncells, 256)),
@@ -1279,47 +1111,68 @@ static int launch_dir(const htr_fields &f, const DMix *mix, const Geo &g, double
    }
 }
 
-// The hybrid sweep along DIR in two parts on two streams (the full RHS with
-// overlap): part 0, the TENO faces into the face buffer of the workspace of
-// stream ts, with the total enthalpy of the workspace of stream hs (formed
-// before); part 1, on stream s, the KG faces and the divergence reading the
-// TENO faces back from the workspace of ts.
-template<class MX, int DIR>
-static int hybrid_part(int part, const htr_fields &f, const DMix *mix, const Geo &g, double RK0, double RK1,
-                       const DtArg &dt, const htr_view &dec, hipStream_t ts, hipStream_t hs, hipStream_t s)
+// Face buffers of the three sweeps of a full right-hand side, one after the
+// other in one workspace
+template<class MX>
+static int64_t rhs_face_base(const Geo &g, int d)
 {
-   if (exec_cells(g) == 0) return HTR_OK;
-   const int64_t nfaces = Faces<DIR>::count(g);
-   if (nfaces*MX::NEQ >= (1ll << 31)) return set_error(HTR_E_UNSUPPORTED, "euler: too many faces");
+   int64_t n = 0;
+   if (d < 2) n += Faces<2>::count(g);
+   if (d < 1) n += Faces<1>::count(g);
+   if (d < 0) n += Faces<0>::count(g);
+   return n*MX::NEQ;
+}
+
+template<class MX, int DIR>
+static int rhs_teno(const htr_fields &f, const DMix *mix, const Geo &g, double RK0, double RK1, const DtArg &dt,
+                    const htr_view &dec, hipStream_t ts, hipStream_t hs, double *F)
+{
    Workspace *tw = workspace(ts), *hw = workspace(hs);
    if (!tw || !hw) return HTR_E_DEVICE;
+   const int64_t nfaces = Faces<DIR>::count(g);
    htr_view hv;
    int rc = enthalpy_view(g, *hw, hv);
+   if (!rc) rc = workspace_faces(*tw, 0, 2*nfaces, teno_doubles<MX>(nfaces));
    if (rc) return rc;
-   if (part == 0) {
-      if ((rc = workspace_faces(*tw, nfaces*MX::NEQ, 2*nfaces, teno_doubles<MX>(nfaces)))) return rc;
-      return teno_faces<MX, DIR>(f, mix, g, hv, RK0, RK1, dt, *tw, nfaces, tw->faces, dec, ts);
-   }
-   if (tw->faces_cap < nfaces*MX::NEQ) return set_error(HTR_E_ARG, "euler: TENO part not run");
-   return kg_walks<MX, DIR, false>(f, g, hv, tw->faces, nfaces, dec, s);
+   return teno_faces<MX, DIR>(f, mix, g, hv, RK0, RK1, dt, *tw, nfaces, F, dec, ts);
 }
 
+// The Euler sweeps of a full right-hand side (hybrid or KG), total enthalpy
+// formed before.  part 0: the TENO faces of direction dir, on stream ts (the
+// list and the records in its workspace), into the face buffer of the
+// workspace of s; part 1: KG faces and divergence of the three directions in
+// one pass on s.
 template<class MX>
-int hybrid_part_dispatch(int dir, int part, const htr_fields &f, const DMix *mix, const Geo &g, double RK0, double RK1,
-                         const DtArg &dt, const htr_view &dec, hipStream_t ts, hipStream_t hs, hipStream_t s)
+int rhs_euler_part(int dir, int part, int scheme, const htr_fields &f, const DMix *mix, const Geo &g, double RK0,
+                   double RK1, const DtArg &dt, const htr_view &dec, hipStream_t ts, hipStream_t s)
 {
-   switch (dir) {
-      case 0: return hybrid_part<MX, 0>(part, f, mix, g, RK0, RK1, dt, dec, ts, hs, s);
-      case 1: return hybrid_part<MX, 1>(part, f, mix, g, RK0, RK1, dt, dec, ts, hs, s);
-      case 2: return hybrid_part<MX, 2>(part, f, mix, g, RK0, RK1, dt, dec, ts, hs, s);
-      default: return set_error(HTR_E_ARG, "euler: bad direction");
+   if (exec_cells(g) == 0) return HTR_OK;
+   for (int64_t n : { Faces<0>::count(g), Faces<1>::count(g), Faces<2>::count(g) })
+      if (n*MX::NEQ >= (1ll << 31)) return set_error(HTR_E_UNSUPPORTED, "euler: too many faces");
+   Workspace *w = workspace(s);
+   if (!w) return HTR_E_DEVICE;
+   int rc = workspace_faces(*w, scheme == HTR_EULER_KG ? 0 : rhs_face_base<MX>(g, -1), 0, 0);
+   if (rc) return rc;
+   KGFaces F;
+   for (int d = 0; d < 3; d++) F.f[d] = w->faces ? w->faces + rhs_face_base<MX>(g, d) : nullptr;
+   if (part == 0) {
+      double *Fd = const_cast<double*>(F.f[dir]);
+      switch (dir) {
+         case 0: return rhs_teno<MX, 0>(f, mix, g, RK0, RK1, dt, dec, ts, s, Fd);
+         case 1: return rhs_teno<MX, 1>(f, mix, g, RK0, RK1, dt, dec, ts, s, Fd);
+         default: return rhs_teno<MX, 2>(f, mix, g, RK0, RK1, dt, dec, ts, s, Fd);
+      }
    }
+   htr_view hv;
+   if ((rc = enthalpy_view(g, *w, hv))) return rc;
+   if (scheme == HTR_EULER_KG) return kg_cells<MX, 7, true>(f, g, hv, F, dec, s);
+   return kg_cells<MX, 7, false>(f, g, hv, F, dec, s);
 }
 
-template int hybrid_part_dispatch<MixCP>(int, int, const htr_fields &, const DMix *, const Geo &, double, double,
-                                         const DtArg &, const htr_view &, hipStream_t, hipStream_t, hipStream_t);
-template int hybrid_part_dispatch<MixAir>(int, int, const htr_fields &, const DMix *, const Geo &, double, double,
-                                          const DtArg &, const htr_view &, hipStream_t, hipStream_t, hipStream_t);
+template int rhs_euler_part<MixCP>(int, int, int, const htr_fields &, const DMix *, const Geo &, double, double,
+                                   const DtArg &, const htr_view &, hipStream_t, hipStream_t);
+template int rhs_euler_part<MixAir>(int, int, int, const htr_fields &, const DMix *, const Geo &, double, double,
+                                    const DtArg &, const htr_view &, hipStream_t, hipStream_t);
 
 // Total enthalpy of every cell of the bounds into the stream's workspace
 // (once per RHS; the three sweeps then skip it)
@@ -1350,7 +1203,7 @@ WorkspaceNeed euler_workspace_need(const Geo &g)
 {
    WorkspaceNeed n;
    auto dir = [&](int64_t nfaces) {
-      n.faces = std::max(n.faces, nfaces*MX::NEQ);
+      n.faces += nfaces*MX::NEQ;               // the full right-hand side holds all three
       n.list = std::max(n.list, 2*nfaces);
       n.teno = std::max(n.teno, teno_doubles<MX>(nfaces));
    };

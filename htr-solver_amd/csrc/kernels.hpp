@@ -46,13 +46,15 @@ template<class MX> int enthalpy_launch(const htr_fields &f, const Geo &g, hipStr
 template<class MX> int euler_dispatch(int dir, int scheme, const htr_fields &f, const DMix *mix, const Geo &g,
                                       double RK0, double RK1, const DtArg &dt, const htr_view &dec, hipStream_t s,
                                       bool enthalpy_ready = false);
-// the hybrid sweep in two parts (full RHS with overlap): part 0, the TENO
-// faces into the workspace of stream ts (total enthalpy from the workspace of
-// hs); part 1, on stream s, the KG faces and the divergence reading them back
-template<class MX> int hybrid_part_dispatch(int dir, int part, const htr_fields &f, const DMix *mix, const Geo &g,
-                                            double RK0, double RK1, const DtArg &dt, const htr_view &dec,
-                                            hipStream_t ts, hipStream_t hs, hipStream_t s);
-template<class MX> int diffusion_dispatch(int dir, const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s);
+// the Euler sweeps of a full RHS (hybrid or KG) in parts: part 0, the TENO
+// faces of direction dir on stream ts into the face buffer of the workspace of
+// s; part 1, on s, the KG faces and the divergence of all three directions in
+// one pass (total enthalpy formed before, in the workspace of s)
+template<class MX> int rhs_euler_part(int dir, int part, int scheme, const htr_fields &f, const DMix *mix,
+                                      const Geo &g, double RK0, double RK1, const DtArg &dt, const htr_view &dec,
+                                      hipStream_t ts, hipStream_t s);
+// dirs: one direction (1 x, 2 y, 4 z) or 7, all three in the order z, y, x
+template<class MX> int diffusion_dispatch(int dirs, const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s);
 template<class MX> int properties_launch(const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s);
 template<class MX> int conserved_launch(const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s);
 template<class MX> int primitive_launch(const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s);
@@ -103,27 +105,5 @@ void prof_end(hipStream_t s);
 
 // "name_x", "name_y", "name_z"
 #define HTR_DIR_NAME(base, dir) ((dir) == 0 ? base "_x" : (dir) == 1 ? base "_y" : base "_z")
-
-// Faces per segment of the y and z line walks (KG and diffusion): the
-// longest of 64, 32, 16, 8 that still gives at least 2^18 threads (16 waves
-// per CU), since a longer segment repeats less warm-up but a short rect then
-// leaves CUs idle.  HTR_WALK_SEGMENT="Lx,Ly,Lz" fixes it (tuning; entry 0
-// is unused: the x sweeps take wave-wide rows).
-static inline int walk_segment(int dir, int64_t nlines, int64_t faces_per_line)
-{
-   static int fixed[3] = { -1, -1, -1 };
-   if (fixed[0] < 0) {
-      int v[3] = { 0, 0, 0 };
-      if (const char *e = getenv("HTR_WALK_SEGMENT")) {
-         int a, b, c;
-         if (sscanf(e, "%d,%d,%d", &a, &b, &c) == 3 && a > 0 && b > 0 && c > 0) { v[0] = a; v[1] = b; v[2] = c; }
-      }
-      fixed[1] = v[1]; fixed[2] = v[2]; fixed[0] = v[0];
-   }
-   if (fixed[dir] > 0) return fixed[dir];
-   int L = 64;
-   while (L > 8 && nlines*((faces_per_line + L - 1)/L) < (int64_t(1) << 18)) L /= 2;
-   return L;
-}
 
 } // namespace htr

@@ -146,9 +146,8 @@ HD const double *cp_range(const DSpec &s, double T)
 // coefficients come through scalar loads and enter as scalar operands.  A wave
 // that straddles a switch (and a mixture too large to hold its species'
 // ranges) gathers.  256^3 air: Roe pass 0.79 -> 0.71 ms per direction (233 ->
-// 147 VGPRs), diffusion species x 1.05 -> 0.86 ms.  The chemistry source
-// evaluates them once per cell and keeps the gathers (0.78 ms; 0.87 ms this
-// way, for a wave less per SIMD).
+// 147 VGPRs).  The chemistry source evaluates them once per cell and keeps the
+// gathers (0.78 ms; 0.87 ms this way, for a wave less per SIMD).
 template<int NS, class M, class F>
 HD void species_loop(const M &m, double T, F f)
 {
@@ -163,14 +162,21 @@ HD void species_loop(const M &m, double T, F f)
          one = one && (hi == 0 || hi == all) && (lo == 0 || lo == all);
          r[i] = hi ? 0 : lo ? 1 : 2;
       }
+      // one species' coefficients at a time, in scalar or vector registers
       if (one) {
 #pragma unroll
          for (int i = 0; i < NS; i++) {
             f(i, m.sp[i], m.sp[i].cp[r[i]]);
-            __builtin_amdgcn_sched_barrier(0);   // one species' scalars at a time
+            __builtin_amdgcn_sched_barrier(0);
          }
-         return;
+      } else {
+#pragma unroll
+         for (int i = 0; i < NS; i++) {
+            f(i, m.sp[i], cp_range(m.sp[i], T));
+            __builtin_amdgcn_sched_barrier(0);
+         }
       }
+      return;
    }
 #endif
 #pragma unroll

@@ -310,9 +310,9 @@ def rk_init(fs, nEq, grid=None, stream=None):
 
 def rhs_overlap(on):
     """Scheduling of the hybrid full RHS: True runs each direction's TENO
-    passes on a library side stream, overlapping the chemistry source and the
-    earlier directions' KG walks (same result to the bit); False (the default)
-    runs every launch on the caller's stream."""
+    passes on a library side stream, overlapping the chemistry source (same
+    result to the bit); False (the default) runs every launch on the caller's
+    stream."""
     check(lib().htr_rhs_overlap(1 if on else 0))
 
 

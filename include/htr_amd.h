@@ -332,11 +332,11 @@ int htr_full_rhs_cfl(const htr_grid *g, const htr_fields *f, int scheme, double 
  * with on = 1 each direction's TENO passes run on a side stream of the
  * library (one per direction and caller stream, created at first use or by
  * htr_workspace_reserve, each with its own workspace) while the caller's
- * stream runs the chemistry source and the earlier directions' KG walks;
+ * stream runs the chemistry source; the KG pass follows them all;
  * events order them, and Conserved_t receives its terms in the same order,
  * so the result is the same to the bit.  on = 0: every launch on the caller's
  * stream.  Applies to later calls.  The side streams gain only where the TENO
- * component kernel leaves room on the CUs for the walks' waves; at its full
+ * component kernel leaves room on the CUs for other waves; at its full
  * persistent grid (3 blocks per CU) one stream is faster. */
 int htr_rhs_overlap(int on);
 
