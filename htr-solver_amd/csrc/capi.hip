@@ -253,16 +253,71 @@ static void build_species_reactions(DMix &d)
    d.spr_ptr[d.nSpec] = n;
 }
 
+// the reactions and the species rows as the lanes of the implicit chemistry
+// read them (DMix::rate, prow, rows), after build_species_reactions and
+// derive_species
+static std::vector<DRow> build_kinetics(DMix &d)
+{
+   d.nRows = d.maxEd = d.maxPd = d.maxTb = 0;
+   d.unitNu = 1;
+   for (int k = 0; k < d.nReac; k++) {
+      const DReac &r = d.rc[k];
+      DRate &q = d.rate[k];
+      q = DRate{r.A, 0.0, r.n, r.EovR, rc_info(r), 0, 0, {0, 0, 0}};
+      auto side = [&](int n, const int *id, const float *nu, float (*out)[MAX_REAC], uint32_t &ids, int sign, int bit) {
+         for (int i = 0; i < n; i++) {
+            if (nu[i] != 1.0f && nu[i] != 2.0f) d.unitNu = 0;
+            if (nu[i] == 2.0f) q.info |= 1u << (bit + i);
+            q.sumNu += sign*(double)nu[i];
+            ids |= (uint32_t)id[i] << 8*i;
+            out[i][k] = nu[i];
+         }
+      };
+      side(r.Ne, r.ed_ind, r.ed_nu, d.kEnu, q.eid, -1, 0);
+      side(r.Np, r.pd_ind, r.pd_nu, d.kPnu, q.pid, 1, 4);
+      for (int i = 0; i < r.Ntb; i++) { d.kTid[i][k] = r.tb_ind[i]; d.kTeff[i][k] = r.tb_eff[i]; }
+      d.maxEd = std::max(d.maxEd, r.Ne);
+      d.maxPd = std::max(d.maxPd, r.Np);
+      if (r.kind == REAC_THIRDB) d.maxTb = std::max(d.maxTb, r.Ntb);
+   }
+   for (int s = 0; s < d.nSpec; s++) {
+      d.nRows = std::max(d.nRows, d.spr_ptr[s+1] - d.spr_ptr[s]);
+      for (int r = 0; r < 3; r++)
+         for (int c = 0; c < 12; c++) d.cpT[r][c][s] = d.sp[s].cp[r][c];
+   }
+   std::vector<DRow> rows((size_t)d.nRows*d.nSpec, DRow{0.0f, (uint32_t)d.nReac, 0, 0});
+   for (auto &w : d.prow)
+      for (uint32_t &v : w) v = (uint32_t)d.nReac*0x10001u;
+   for (int s = 0; s < d.nSpec; s++)
+      for (int e = d.spr_ptr[s]; e < d.spr_ptr[s+1]; e++) {
+         const int k = d.spr_reac[e], at = e - d.spr_ptr[s], sh = 16*(at % 2);
+         const float nu = d.spr_nu[e];
+         const uint32_t code = (uint32_t)k | (fabsf(nu) == 2.0f ? 0x2000u : 0u) | (nu < 0.0f ? 0x4000u : 0u);
+         uint32_t &w = d.prow[at/2][s];
+         w = (w & ~(0xffffu << sh)) | code << sh;
+         rows[(size_t)at*d.nSpec + s] = DRow{nu, rc_info(d.rc[k]) | (uint32_t)k, d.rate[k].eid, d.rate[k].pid};
+      }
+   return rows;
+}
+
 static int upload(htr_mix *m)
 {
    int rc = ensure_device();
    if (rc) return rc;
+   std::vector<DRow> rows;
    if (!m->host.constprop) build_species_reactions(m->host);
    for (int i = 0; i < m->host.nSpec; i++) derive_species(m->host.sp[i]);
-   if (!m->host.constprop) derive_transport(m->host);
-   if (!m->dev && hipMalloc(&m->dev, sizeof(DMix)) != hipSuccess)
+   if (!m->host.constprop) {
+      derive_transport(m->host);
+      rows = build_kinetics(m->host);
+   }
+   // the rows follow the mixture in one allocation (a mixture's reactions are
+   // fixed once it is uploaded)
+   const size_t at = DMix::rows_at(), bytes = rows.size()*sizeof(DRow);
+   if (!m->dev && hipMalloc((void **)&m->dev, at + bytes) != hipSuccess)
       return set_error(HTR_E_DEVICE, "mixture allocation failed");
-   if (hipMemcpy(m->dev, &m->host, sizeof(DMix), hipMemcpyHostToDevice) != hipSuccess)
+   if (hipMemcpy(m->dev, &m->host, sizeof(DMix), hipMemcpyHostToDevice) != hipSuccess ||
+       (bytes && hipMemcpy(reinterpret_cast<char*>(m->dev) + at, rows.data(), bytes, hipMemcpyHostToDevice) != hipSuccess))
       return set_error(HTR_E_DEVICE, "mixture upload failed");
    m->finalized = 1;
    return HTR_OK;
@@ -881,8 +936,8 @@ int htr_chem_update(const htr_grid *g, const htr_fields *f, double dt, int preci
    }
    HTR_NEED(Conserved); HTR_NEED(Conserved_t); HTR_NEED(Conserved_t_old); HTR_NEED(temperature);
    switch (kind_of(m)) {
-      case K_AIR: return chem_update_launch<MixAir>(fr, m->dev, geo, dt, precision, ns, m->host.nReac, (hipStream_t)stream);
-      case K_30:  return chem_update_launch<Mix30>(fr, m->dev, geo, dt, precision, ns, m->host.nReac, (hipStream_t)stream);
+      case K_AIR: return chem_update_launch<MixAir>(fr, m->dev, geo, dt, precision, ns, m->host, (hipStream_t)stream);
+      case K_30:  return chem_update_launch<Mix30>(fr, m->dev, geo, dt, precision, ns, m->host, (hipStream_t)stream);
       default: return set_error(HTR_E_UNSUPPORTED, "implicit chemistry: no kernel instance for %d species", m->host.nSpec);
    }
 }

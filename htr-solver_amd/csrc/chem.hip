@@ -5,6 +5,10 @@
 // src/prometeo_chem.cc:36-71 (task loop), src/Utils/math_utils.hpp:87-438
 // (LUdec, Rosenbrock: FD Jacobian, step, itercheck, stepcheck).
 //
+// With 64 lanes per cell (the 30-species mechanism's default) chem_wave.hpp
+// integrates a cell per wave, in registers; with fewer lanes (small mechanisms,
+// where 64 lanes would idle; bit-identical) this file's groups do:
+//
 // A group of L lanes of one wave integrates one cell (64/L cells per wave);
 // the groups pull cells from an atomic work queue, so cells with many steps
 // do not hold others back.  The cell's Jacobian, its LU factors and the
@@ -34,10 +38,7 @@
 //                     of the solution; a solve whose refinement stalls makes
 //                     the step fall back to an FP64 LU of the same matrix,
 //                     factorised in place of the Jacobian (which is then
-//                     formed again if the step is retried).  With 64 lanes per
-//                     cell the refinement runs in registers (one row per lane,
-//                     operands broadcast by readlane); the rounding order of
-//                     its triangular solves is free, the refinement fixes it.
+//                     formed again if the step is retried).
 //
 // Two Jacobians (HTR_CHEM_JAC_ANALYTIC or-ed into the precision):
 //   central differences  the reference's, 2 nEq right-hand sides;
@@ -51,18 +52,9 @@
 //                        per step instead of 2 nEq + 1 right-hand sides.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "chem_wave.hpp"
 
 namespace htr {
-
-// LDS synchronisation of a lane group inside one wave: LDS operations of a
-// wave complete in order; the fences keep the compiler from moving them
-// across and wait for the outstanding ones.
-__device__ __forceinline__ void gsync()
-{
-   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-   __builtin_amdgcn_wave_barrier();
-   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
 
 // Offsets (in doubles) of one cell's LDS region.
 template<class MX, int PREC>
@@ -403,16 +395,6 @@ struct ChemGroup {
       jac_valid = true;
    }
 
-   // power of two nearest to 1/a (exact scaling)
-   __device__ __forceinline__ static double pow2_inv(double a)
-   {
-      if (!(a > 0.0) || !(a < 1.0e308)) return 1.0;
-      // a = m 2^e with m in [0.5, 1): e from the biased exponent (normal a)
-      const int be = (int)((__double_as_longlong(a) >> 52) & 0x7ff);
-      if (be == 0) return 1.0;
-      return ldexp(1.0, -(be - 1022));
-   }
-
    // LUdec::ludcmp (math_utils.hpp:87-155) of the N x N column-major matrix M
    template<typename T_>
    __device__ __forceinline__ void ludcmp(T_ *M)
@@ -469,73 +451,6 @@ struct ChemGroup {
       }
    }
 
-   // ludcmp with one row per lane (L == 64 >= N): lane i holds row i of the
-   // matrix in registers and keeps it; its current position (the row index
-   // after the interchanges so far) is tracked instead of moving the data.
-   // Per column the candidates are the rows at positions >= j, the pivot the
-   // last position attaining the maximum scaled magnitude (the reference's
-   // `>=' scan), the pivot row is broadcast by readlane, and every entry
-   // receives the same products in the same order as ludcmp above, so the
-   // factors and the pivot indices are the same.  The factors are written to
-   // Mout in the reference's layout (row = final position).  The row of lane
-   // i is a(k) for k < N.
-   template<typename T_, typename F_>
-   __device__ __forceinline__ void ludcmp_reg(T_ *Mout, F_ a)
-   {
-      static_assert(L == 64 && N <= 64, "one row per lane");
-      int *piv = ind();
-      const bool act = lane < N;
-      T_ row[N];
-#pragma unroll
-      for (int k = 0; k < N; k++) row[k] = act ? a(k) : (T_)0;
-      T_ big = 0;
-#pragma unroll
-      for (int k = 0; k < N; k++) { const T_ x = fabs(row[k]); big = (big < x) ? x : big; }
-      const T_ vvi = (T_)1/big;
-      int pos = lane;
-#pragma unroll
-      for (int j = 0; j < N; j++) {
-         // pivot: the last position >= j with the largest vv |M(i, j)|
-         const T_ dum = vvi*fabs(row[j]);
-         const bool cand = act && pos >= j && ((double)dum >= -1.0);
-         double best = cand ? (double)dum : -1.0;
-         int bp = cand ? pos : -1;
-#pragma unroll
-         for (int o = 32; o > 0; o >>= 1) {
-            const double ob = __shfl_xor(best, o, 64);
-            const int op = __shfl_xor(bp, o, 64);
-            if (ob > best || (ob == best && op > bp)) { best = ob; bp = op; }
-         }
-         const int imax = __builtin_amdgcn_readfirstlane((bp < 0) ? j : bp);
-         const unsigned long long mw = __ballot(act && pos == imax);
-         const unsigned long long mj = __ballot(act && pos == j);
-         const int P = __ffsll((long long)mw) - 1, Pj = __ffsll((long long)mj) - 1;
-         if (lane == P) pos = j;
-         else if (lane == Pj) pos = imax;
-         if (lane == 0) piv[j] = imax;
-         T_ pv = (sizeof(T_) == 8) ? (T_)rdlane((double)row[j], P) : (T_)rdlanef((float)row[j], P);
-         if (pv == (T_)0) {
-            pv = (T_)1.0e-20;
-            if (lane == P) row[j] = pv;
-         }
-         if (j != N - 1) {
-            const T_ dv = (T_)1/pv;
-            const bool below = act && pos > j;
-            if (below) row[j] *= dv;
-#pragma unroll
-            for (int k = j + 1; k < N; k++) {
-               const T_ ujk = (sizeof(T_) == 8) ? (T_)rdlane((double)row[k], P) : (T_)rdlanef((float)row[k], P);
-               if (below) row[k] -= row[j]*ujk;
-            }
-         }
-      }
-      if (act) {
-#pragma unroll
-         for (int k = 0; k < N; k++) Mout[pos + k*N] = row[k];
-      }
-      gsync();
-   }
-
    // LUdec::lubksb (math_utils.hpp:157-188): permutation, forward
    // substitution column by column (each entry receives its products in the
    // reference's order), back substitution row by row by one lane in the
@@ -572,16 +487,11 @@ struct ChemGroup {
       if (PREC == HTR_CHEM_FP64) {
          double *M = reinterpret_cast<double*>(A);
          const double *J = Jm();
-         if constexpr (L == 64 && N <= 64) {
-            const int i = lane;
-            ludcmp_reg<double>(M, [&](int k) { double x = -J[i + k*N]; if (k == i) x += d; return x; });
-         } else {
-            for (int e = lane; e < N*N; e += L) M[e] = -J[e];
-            gsync();
-            for (int i = lane; i < N; i += L) M[i + i*N] += d;
-            gsync();
-            ludcmp<double>(M);
-         }
+         for (int e = lane; e < N*N; e += L) M[e] = -J[e];
+         gsync();
+         for (int i = lane; i < N; i += L) M[i + i*N] += d;
+         gsync();
+         ludcmp<double>(M);
       } else {
          // equilibrate by powers of two (rows, then columns) before rounding
          // to FP32
@@ -600,24 +510,12 @@ struct ChemGroup {
          }
          gsync();
          float *M = reinterpret_cast<float*>(A);
-         if constexpr (L == 64 && N <= 64) {
-            const int i = lane;
-            const double rsi = (i < N) ? rs[i] : 0.0;
-            ludcmp_reg<float>(M, [&](int k) { return (float)(rsi*(-J[i + k*N] + ((i == k) ? d : 0.0))*cs[k]); });
-         } else {
-            for (int e = lane; e < N*N; e += L) {
-               const int i = e % N, j = e/N;
-               M[e] = (float)(rs[i]*(-J[e] + ((i == j) ? d : 0.0))*cs[j]);
-            }
-            gsync();
-            ludcmp<float>(M);
+         for (int e = lane; e < N*N; e += L) {
+            const int i = e % N, j = e/N;
+            M[e] = (float)(rs[i]*(-J[e] + ((i == j) ? d : 0.0))*cs[j]);
          }
-         if (L == 64 && N <= 64) {
-            // reciprocal pivots of the register refinement
-            double *ud = v(Lay::VV);
-            for (int i = lane; i < N; i += L) ud[i] = (double)(1.0f/M[i + i*N]);
-            gsync();
-         }
+         gsync();
+         ludcmp<float>(M);
          lu64 = false;
       }
    }
@@ -637,88 +535,11 @@ struct ChemGroup {
       fallbacks++;
    }
 
-   // value of v in lane l of the wave (l uniform)
-   __device__ __forceinline__ static double rdlane(double x, int l)
-   {
-      const long long b = __double_as_longlong(x);
-      const int lo = __builtin_amdgcn_readlane((int)b, l);
-      const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-      return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-   }
-
-   __device__ __forceinline__ static float rdlanef(float x, int l)
-   {
-      return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
-   }
-
-   // FP32_IR refinement with one row per lane (L == 64 >= N): the solution
-   // and the FP64 residual in registers, the correction solved in FP32 with
-   // the FP32 factors (read from LDS, reciprocal pivots formed once per
-   // factorisation), operands broadcast by readlane.  Returns false when the
-   // refinement stalls (b then holds the right-hand side).
-   __device__ __forceinline__ bool solve_ir_reg(double *b, double dt)
-   {
-      const float *M = reinterpret_cast<const float*>(A);
-      const double *J = Jm();
-      const double *rs = v(Lay::RS), *cs = v(Lay::CS), *ud = v(Lay::VV);
-      const int *piv = ind();
-      const int i = lane;
-      const bool act = i < N;
-      const double d = 1.0/((1.0/2.0)*dt);
-      const double rb = act ? b[i] : 0.0;
-      const double rsi = act ? rs[i] : 0.0, csi = act ? cs[i] : 0.0;
-      double xk = 0.0, prev = 0.0;
-      bool done = false;
-      for (int it = 0; it < 9 && !done; it++) {
-         double r = rb;
-         if (it > 0) {
-            for (int j = 0; j < N; j++) {
-               const double xj = rdlane(xk, j);
-               if (act) r -= (((i == j) ? d : 0.0) - J[i + j*N])*xj;
-            }
-         }
-         float rf = (float)(r*rsi);
-         for (int k = 0; k < N; k++) {          // row interchanges, in order
-            const int ip = __builtin_amdgcn_readfirstlane(piv[k]);
-            const float vk = rdlanef(rf, k), vp = rdlanef(rf, ip);
-            if (i == k) rf = vp;
-            if (i == ip) rf = vk;
-         }
-         for (int k = 0; k < N - 1; k++) {      // unit lower triangle
-            const float bk = rdlanef(rf, k);
-            if (act && i > k) rf -= M[i + k*N]*bk;
-         }
-         for (int k = N - 1; k >= 0; k--) {     // upper triangle
-            const float xkk = rdlanef(rf, k)*(float)ud[k];
-            if (i == k) rf = xkk;
-            else if (act && i < k) rf -= M[i + k*N]*xkk;
-         }
-         const double ci = act ? csi*(double)rf : 0.0;
-         xk += ci;
-         const double nc = gmax(fabs(ci)), nx = gmax(fabs(xk));
-         if (it == 0) { prev = nc; continue; }
-         if (!(nc > 1e-15*nx)) done = true;
-         else if (!(nc < 0.5*prev)) break;
-         prev = nc;
-      }
-      if (done && act) b[i] = xk;
-      gsync();
-      return done;
-   }
-
    // b <- A^-1 b
    __device__ __forceinline__ void solve(double *b, double dt)
    {
       if (PREC == HTR_CHEM_FP64) { lubksb<double, double>(reinterpret_cast<double*>(A), b); return; }
       if (lu64) { lubksb<double, double>(Jm(), b); return; }
-      if (L == 64 && N <= 64) {
-         if (!solve_ir_reg(b, dt)) {
-            // refinement stalled: FP64 LU of the same matrix for this step
-            factor64_in_place(dt);
-            lubksb<double, double>(Jm(), b);
-         }
-         return;
-      }
       const float *M = reinterpret_cast<const float*>(A);
       const double *J = Jm();
       const double *rs = v(Lay::RS), *cs = v(Lay::CS);
@@ -918,6 +739,7 @@ template<class MX, int PREC, int L>
 static int chem_launch_l(const htr_fields &f, const DMix *mix, const Geo &g, double dt, const htr_view &nsteps,
                          Workspace &w, int nreac, int64_t n, bool aj, hipStream_t s)
 {
+   static_assert(L < 64, "64 lanes per cell: chem_wave_kernel");
    using Lay = ChemLayout<MX, PREC>;
    const int cd = Lay::cell_doubles(nreac, aj);
    const size_t shm = (size_t)(64/L)*cd*sizeof(double);
@@ -933,23 +755,42 @@ static int chem_launch_l(const htr_fields &f, const DMix *mix, const Geo &g, dou
    return check_launch("chem_group_kernel");
 }
 
+template<class MX, int PREC, bool AJ>
+static int chem_launch_wave(const htr_fields &f, const DMix *mix, const Geo &g, double dt, const htr_view &nsteps,
+                            Workspace &w, const DMix &host, int64_t n, hipStream_t s)
+{
+   const WaveLayout<MX, PREC, AJ> L(host.nReac, host.maxEd, host.maxPd);
+   const size_t shm = (size_t)L.total*sizeof(double);
+   if (shm > 160*1024) return set_error(HTR_E_UNSUPPORTED, "chem: %zu B of LDS per cell", shm);
+   int per_cu = g_chem_blocks_per_cu;
+   if (per_cu == 0) per_cu = std::max(1, std::min(16, (int)((160*1024)/shm)));
+   const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(n, (int64_t)256*per_cu));
+   HTR_LAUNCH(PREC == HTR_CHEM_FP64 ? (AJ ? "chem_update_fp64_aj" : "chem_update_fp64")
+                                    : (AJ ? "chem_update_fp32ir_aj" : "chem_update_fp32ir"),
+              (chem_wave_kernel<MX, PREC, AJ>), dim3(blocks), dim3(AJ ? 64 : 64*CHEM_FD_WAVES), shm, s, f, mix, g, dt,
+              nsteps, w.counter, w.counter + 3, n);
+   return check_launch("chem_wave_kernel");
+}
+
 template<class MX, int PREC>
 static int chem_launch_p(const htr_fields &f, const DMix *mix, const Geo &g, double dt, const htr_view &nsteps,
-                         Workspace &w, int nreac, int64_t n, bool aj, hipStream_t s)
+                         Workspace &w, const DMix &host, int64_t n, bool aj, hipStream_t s)
 {
    int lanes = g_chem_lanes;
    if (lanes == 0) lanes = (MX::NS >= 16) ? 64 : 16;
+   const int nreac = host.nReac;
    switch (lanes) {
       case 8:  return chem_launch_l<MX, PREC, 8>(f, mix, g, dt, nsteps, w, nreac, n, aj, s);
       case 16: return chem_launch_l<MX, PREC, 16>(f, mix, g, dt, nsteps, w, nreac, n, aj, s);
       case 32: return chem_launch_l<MX, PREC, 32>(f, mix, g, dt, nsteps, w, nreac, n, aj, s);
-      default: return chem_launch_l<MX, PREC, 64>(f, mix, g, dt, nsteps, w, nreac, n, aj, s);
+      default: return aj ? chem_launch_wave<MX, PREC, true>(f, mix, g, dt, nsteps, w, host, n, s)
+                         : chem_launch_wave<MX, PREC, false>(f, mix, g, dt, nsteps, w, host, n, s);
    }
 }
 
 template<class MX>
 int chem_update_launch(const htr_fields &f, const DMix *mix, const Geo &g, double dt, int precision,
-                       const htr_view &nsteps, int nreac, hipStream_t s)
+                       const htr_view &nsteps, const DMix &host, hipStream_t s)
 {
    const int64_t n = exec_cells(g);
    if (n == 0) return HTR_OK;
@@ -959,8 +800,8 @@ int chem_update_launch(const htr_fields &f, const DMix *mix, const Geo &g, doubl
    if (int rc0 = zero_counters(w.counter, s)) return rc0;      // failures and the cell queue
    const bool aj = (precision & HTR_CHEM_JAC_ANALYTIC) != 0;
    const int prec = precision & ~HTR_CHEM_JAC_ANALYTIC;
-   int rc = (prec == HTR_CHEM_FP64) ? chem_launch_p<MX, HTR_CHEM_FP64>(f, mix, g, dt, nsteps, w, nreac, n, aj, s)
-                                    : chem_launch_p<MX, HTR_CHEM_FP32_IR>(f, mix, g, dt, nsteps, w, nreac, n, aj, s);
+   int rc = (prec == HTR_CHEM_FP64) ? chem_launch_p<MX, HTR_CHEM_FP64>(f, mix, g, dt, nsteps, w, host, n, aj, s)
+                                    : chem_launch_p<MX, HTR_CHEM_FP32_IR>(f, mix, g, dt, nsteps, w, host, n, aj, s);
    if (rc) return rc;
    int fails = 0;
    if (hipMemcpyAsync(&fails, w.counter, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -971,8 +812,8 @@ int chem_update_launch(const htr_fields &f, const DMix *mix, const Geo &g, doubl
 }
 
 template int chem_update_launch<MixAir>(const htr_fields &, const DMix *, const Geo &, double, int, const htr_view &,
-                                        int, hipStream_t);
+                                        const DMix &, hipStream_t);
 template int chem_update_launch<Mix30>(const htr_fields &, const DMix *, const Geo &, double, int, const htr_view &,
-                                       int, hipStream_t);
+                                       const DMix &, hipStream_t);
 
 } // namespace htr

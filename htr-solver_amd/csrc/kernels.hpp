@@ -64,7 +64,7 @@ int ducros_launch(const htr_fields &f, const Geo &g, double vorticityScale, hipS
 template<class MX> int chem_source_launch(const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s,
                                           bool zero = false);
 template<class MX> int chem_update_launch(const htr_fields &f, const DMix *mix, const Geo &g, double dt,
-                                          int precision, const htr_view &nsteps, int nreac, hipStream_t s);
+                                          int precision, const htr_view &nsteps, const DMix &host, hipStream_t s);
 template<class MX> int spectral_radius_launch(const htr_fields &f, const DMix *mix, const Geo &g,
                                               double *result, hipStream_t s);
 // the same maximum written to device memory, partials in a file-scope device

@@ -61,6 +61,14 @@ struct DReac {
 
 constexpr int MAX_SPR  = MAX_REAC*(MAX_ED + MAX_PD);
 
+// An entry of the species rows of the stoichiometry, for the lane-per-species
+// passes of the implicit chemistry: reaction, signed coefficient, and the
+// reaction's species (a byte each), so that a row's reads depend on nothing.
+struct alignas(16) DRow { float nu; uint32_t info, eid, pid; };   // info: reaction | rc_info
+// A reaction as the lane-per-reaction passes read it.  info: rc_info, and in
+// the low byte the educts (bits 0-3) and products (4-7) of coefficient 2
+struct alignas(16) DRate { double A, sumNu; float n, EovR; uint32_t info, eid, pid, pad[3]; };
+
 // temperature-independent transport factors of a species and of a pair (i, j)
 struct DTran { double mu, fV, zrot, isk; };
 struct DPair { double w4, iw8, kT, iD; };
@@ -84,7 +92,33 @@ struct DMix {
    int     spr_ptr[MAX_SP + 1];
    int16_t spr_reac[MAX_SPR];
    float   spr_nu[MAX_SPR];
+   // The same rows and the reactions field by field, so that the lanes of a
+   // wave (a lane per species, a lane per reaction) read consecutive words:
+   // entry k of species s is rows()[k*nSpec + s], k < spr_ptr[s+1] - spr_ptr[s]
+   // <= nRows (behind the mixture, in its allocation); coefficients of a
+   // species' polynomials are cpT[range][c][s].
+   int     nRows, maxEd, maxPd, maxTb;
+   int     unitNu;             // every stoichiometric coefficient is 1 or 2
+   // with unitNu, two entries of a species' row in a word: reaction, doubled
+   // (0x2000), negative (0x4000); past the row's end the reaction is nReac
+   uint32_t prow[MAX_SPR/2 + 16][MAX_SP];
+   double  cpT[3][12][MAX_SP];
+   DRate   rate[MAX_REAC];
+   float   kEnu[MAX_ED][MAX_REAC], kPnu[MAX_PD][MAX_REAC];
+   int     kTid[MAX_TB][MAX_REAC];
+   float   kTeff[MAX_TB][MAX_REAC];
+   __host__ __device__ static size_t rows_at();
+   __device__ const DRow *rows() const { return reinterpret_cast<const DRow*>(reinterpret_cast<const char*>(this) + rows_at()); }
 };
+__host__ __device__ inline size_t DMix::rows_at() { return (sizeof(DMix) + 255) & ~(size_t)255; }
+
+// arity of a reaction in the upper half of a word: educts, products, third
+// bodies that act (4 bits each), reversible
+inline uint32_t rc_info(const DReac &r)
+{
+   const int tb = (r.kind == REAC_THIRDB) ? r.Ntb : 0;
+   return ((uint32_t)r.Ne << 16) | ((uint32_t)r.Np << 20) | ((uint32_t)tb << 24) | (r.has_backward ? 1u << 28 : 0u);
+}
 
 #define HD __host__ __device__ inline
 
@@ -197,8 +231,9 @@ inline void derive_species(DSpec &s)
    s.tLo = (double)s.TSwitch1;
 }
 
-// polynomials on the coefficients c of a range (Species.inl:35-160)
-HD double poly_cp(const DSpec &s, const double *c, double T, double Tinv)
+// polynomials on the coefficients c of a range (Species.inl:35-160); S holds rOvW
+template<class S>
+HD double poly_cp(const S &s, const double *c, double T, double Tinv)
 {
    const double poly = c[3] + T*(c[4] + T*(c[5] + T*c[6]));
    return s.rOvW*(c[0]*Tinv*Tinv + c[1]*Tinv + c[2] + T*poly);
@@ -210,7 +245,8 @@ HD double poly_free_enthalpy(const double *c, double T, double Tinv, double logT
    return G - 0.5*T*(c[3] + T*(c[9] + T*(c[10] + 0.1*T*c[6])));
 }
 
-HD double poly_enthalpy(const DSpec &s, const double *c, double T, double Tinv, double logT)
+template<class S>
+HD double poly_enthalpy(const S &s, const double *c, double T, double Tinv, double logT)
 {
    const double E = -c[0]*Tinv + c[1]*logT + c[7] + T*(c[2] + T*(c[3]*0.50 + T*(c[9] + T*(c[5]*0.25 + c[11]*T))));
    return E*s.rOvW;
