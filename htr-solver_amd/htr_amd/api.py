@@ -5,6 +5,7 @@ src/prometeo_types.h:48-114), a Mixture and the task's scalar arguments, and
 runs the corresponding C-ABI entry point on the current HIP stream.
 """
 import ctypes as C
+import struct
 
 import numpy as np
 import torch
@@ -101,6 +102,13 @@ class Mixture:
                 lib().htr_mix_destroy(self.h)
         except Exception:
             pass
+
+
+# the views of htr_fields in the order of the struct, without the profiles that end it
+FIELD_ORDER = tuple("%s%d" % (k, d) for k in ("nType", "m_e", "m_d", "m_s") for d in range(3)) + (
+    "rho", "mu", "lam", "Di", "SoS", "pressure", "temperature", "MassFracs", "MolarFracs", "velocity", "Conserved",
+    "Conserved_old", "Conserved_t", "Conserved_t_old", "shockSensor0", "shockSensor1", "shockSensor2", "DucrosSensor")
+_PACK_FIELDS = struct.Struct("=" + "qqqqq" * len(FIELD_ORDER)).pack_into
 
 
 def make_grid(n, lo=(0, 0, 0), hi=None, bounds_lo=(0, 0, 0)):
@@ -208,17 +216,32 @@ class FieldSet:
         return v
 
     def c(self):
+        """The htr_fields of the call, from the tensors as they are now (they
+        may be exchanged or resized between calls).  All views are packed in
+        one go: set field by field through ctypes they took more of the host's
+        time than the launches of a call, and small boxes wait for the host
+        (a stage of a 200^2 vortex, nine calls: 296 us, packed 178)."""
+        t = self.t
+        lo0, lo1, lo2 = self.bounds_lo
+        at_origin = not (lo0 or lo1 or lo2)
+        vals = []
+        put = vals.extend
+        for k in FIELD_ORDER:
+            x = t[k]
+            s = x.stride()
+            if len(s) == 4:
+                sc, sz, sy, sx = s
+            else:
+                sz, sy, sx = s
+                sc = 0
+            p = x.data_ptr()
+            if not at_origin:
+                p -= (lo0 * sx + lo1 * sy + lo2 * sz) * x.element_size()
+            put((p, sx, sy, sz, sc))
         f = Fields()
-        for d in range(3):
-            f.nType[d] = self.view("nType%d" % d)
-            f.m_e[d] = self.view("m_e%d" % d)
-            f.m_d[d] = self.view("m_d%d" % d)
-            f.m_s[d] = self.view("m_s%d" % d)
-            f.shockSensor[d] = self.view("shockSensor%d" % d)
-        for k in SCALARS + tuple(VECTORS):
-            setattr(f, k, self.view(k))
+        _PACK_FIELDS(f, 0, *vals)
         for k in PROFILES:
-            if k in self.t:
+            if k in t:
                 setattr(f, k, self.view(k))
         return f
 
