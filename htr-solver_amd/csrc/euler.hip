@@ -441,29 +441,33 @@ __device__ inline void store_face(double *__restrict__ F, int64_t nfaces, uint32
 // rows together: for the y and z sweeps a block's faces are a tile of 64
 // x-cells x 8 faces along the sweep x 8 cells of the remaining direction
 // (a wave takes one x-row of the tile); for the x sweep, whose stencil runs
-// along the row, 4096 consecutive face ids.
-constexpr int CLS_PER_THREAD = 16;
+// along the row, 4096 consecutive face ids.  A box too small to give every CU
+// a block of that size takes tiles of 1024 or 256 faces, four or one a thread
+// (a block's atomic costs 12 ns in line with the others', a round of dependent
+// loads 1 us): ten blocks of sixteen rounds took 19.8 us for the x faces of a
+// 200^2 box, in tiles of 256 it takes 4.0; 5001-cell tube 16.8 -> 3.5 us.
 
-template<int DIR, int TX = 16, int TJ = 32>
+template<int DIR, int PT, int TX = 16, int TJ = 2*PT>
 struct ClsTiles {
    static constexpr int B = Faces<DIR>::B;
-   static constexpr int TB = 4096/(TX*TJ);
-   static_assert(TX*TJ*TB == 4096 && (TX & (TX - 1)) == 0 && (TJ & (TJ - 1)) == 0, "tile of 4096 faces");
+   static constexpr uint32_t FACES = 256*PT;
+   static constexpr int TB = FACES/(TX*TJ);
+   static_assert(TX*TJ*TB == FACES && (TX & (TX - 1)) == 0 && (TJ & (TJ - 1)) == 0, "tile of 256 PT faces");
    static constexpr int LX = (TX == 64) ? 6 : (TX == 32) ? 5 : (TX == 16) ? 4 : 3;
-   static constexpr int LJ = (TJ == 64) ? 6 : (TJ == 32) ? 5 : (TJ == 16) ? 4 : (TJ == 8) ? 3 : 2;
+   static constexpr int LJ = (TJ == 64) ? 6 : (TJ == 32) ? 5 : (TJ == 16) ? 4 : (TJ == 8) ? 3 : (TJ == 4) ? 2 : 1;
    __host__ __device__ static uint32_t ntx(const Geo &g) { return ((uint32_t)g.esz[0] + TX - 1u)/TX; }
    __host__ __device__ static uint32_t ntj(const Geo &g) { return ((uint32_t)g.esz[DIR] + TJ)/TJ; }
    __host__ __device__ static uint32_t ntb(const Geo &g) { return ((uint32_t)g.esz[B] + TB - 1u)/TB; }
    static int64_t blocks(const Geo &g, int64_t nfaces)
    {
-      if (DIR == 0) return (nfaces + 4095)/4096;
+      if (DIR == 0) return (nfaces + FACES - 1)/FACES;
       return (int64_t)ntx(g)*ntj(g)*ntb(g);
    }
-   // face id of element e (0..4095) of block b; false past the rect
+   // face id of element e (0..FACES - 1) of block b; false past the rect
    __device__ static bool face(const Geo &g, int64_t nfaces, uint32_t b, uint32_t e, uint32_t &fid)
    {
       if (DIR == 0) {
-         const int64_t id = (int64_t)b*4096 + e;
+         const int64_t id = (int64_t)b*FACES + e;
          fid = (uint32_t)id;
          return id < nfaces;
       }
@@ -476,7 +480,7 @@ struct ClsTiles {
    }
 };
 
-template<class MX, int DIR>
+template<class MX, int DIR, int PT>
 __global__ void __launch_bounds__(256)
 euler_classify_kernel(const htr_fields f, const Geo g, int64_t nfaces, int32_t *__restrict__ list,
                       int *__restrict__ counter)
@@ -486,12 +490,12 @@ euler_classify_kernel(const htr_fields f, const Geo g, int64_t nfaces, int32_t *
    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
    uint32_t flags = 0;
    int before = 0;                    // TENO faces of this wave in earlier rounds
-   uint64_t masks[CLS_PER_THREAD];
+   uint64_t masks[PT];
 #pragma unroll
-   for (int k = 0; k < CLS_PER_THREAD; k++) {
+   for (int k = 0; k < PT; k++) {
       uint32_t fid;
       bool teno = false;
-      if (ClsTiles<DIR>::face(g, nfaces, blockIdx.x, k*256 + threadIdx.x, fid)) {
+      if (ClsTiles<DIR, PT>::face(g, nfaces, blockIdx.x, k*256 + threadIdx.x, fid)) {
          const P3 q = Faces<DIR>::cell(g, f, fid);
          teno = !hybrid_kg<DIR>(f, g, q, ld<int>(f.nType[DIR], q));
       }
@@ -510,10 +514,10 @@ euler_classify_kernel(const htr_fields f, const Geo g, int64_t nfaces, int32_t *
    for (int w = 0; w < wv; w++) base += wave_count[w];
    const uint64_t lt = (1ull << lane) - 1ull;
 #pragma unroll
-   for (int k = 0; k < CLS_PER_THREAD; k++) {
+   for (int k = 0; k < PT; k++) {
       if (flags & (1u << k)) {
          uint32_t fid = 0;
-         ClsTiles<DIR>::face(g, nfaces, blockIdx.x, k*256 + threadIdx.x, fid);
+         ClsTiles<DIR, PT>::face(g, nfaces, blockIdx.x, k*256 + threadIdx.x, fid);
          list[base + __popcll(masks[k] & lt)] = (int32_t)fid;
       }
       base += __popcll(masks[k]);
@@ -1035,8 +1039,14 @@ static int teno_faces(const htr_fields &f, const DMix *mix, const Geo &g, const 
 {
    int rc = zero_counters(w.counter, s);        // TENO list and limiter list counts
    if (rc) return rc;
-   HTR_LAUNCH(HTR_DIR_NAME("euler_classify", DIR), (euler_classify_kernel<MX, DIR>),
-              dim3((unsigned)ClsTiles<DIR>::blocks(g, nfaces)), dim3(256), 0, s, f, g, nfaces, w.list, w.counter + 1);
+   auto classify = [&](auto pt) {
+      constexpr int PT = decltype(pt)::value;
+      HTR_LAUNCH(HTR_DIR_NAME("euler_classify", DIR), (euler_classify_kernel<MX, DIR, PT>),
+                 dim3((unsigned)ClsTiles<DIR, PT>::blocks(g, nfaces)), dim3(256), 0, s, f, g, nfaces, w.list, w.counter + 1);
+   };
+   if (nfaces >= 256*4096)      classify(std::integral_constant<int, 16>());
+   else if (nfaces >= 256*1024) classify(std::integral_constant<int, 4>());
+   else                         classify(std::integral_constant<int, 1>());
    if ((rc = check_launch("euler_classify_kernel"))) return rc;
    return launch_teno<MX, DIR, HTR_EULER_TENO, true>(f, mix, g, hv, RK0, RK1, dt, w, nfaces, F, dec, s);
 }
