@@ -18,10 +18,12 @@
 //     other three form the production rates of the columns before, each the
 //     pair of one column at once.
 // 30 species, 180 reactions, against 64 lanes of the group kernel before:
-// 12^3 cells, FP64, central differences 755 -> 159 ms; 20^3 cells, FP32 and
-// refinement, analytic Jacobian 423 -> 137 ms; 32^3 cells 5150 -> 2510 ms (FP64,
-// differences), 1435 -> 553 ms (FP64, analytic), 1298 -> 643 ms (refined,
-// analytic).
+// 12^3 cells, FP64, central differences 1033 -> 197 ms; 20^3 cells, FP32 and
+// refinement, analytic Jacobian 576 -> 155 ms; 32^3 cells 5150 -> 2470 ms (FP64,
+// differences), 1435 -> 571 ms (FP64, analytic), 1298 -> 539 ms (refined,
+// analytic).  Still bound by latency: of 220000 cycles of a step with the
+// analytic Jacobian the factorisation takes 45000, the solves 73000, the
+// Jacobian 40000; with differences the Newtons' chain takes 184000 of 475000.
 #pragma once
 #include "common.hpp"
 #include "kernels.hpp"
@@ -73,6 +75,24 @@ __device__ __forceinline__ double wave_dmax(double x)
 #endif
    return rdlane(x, 63);
 }
+
+// maximum of a 32-bit key: one instruction a step
+__device__ __forceinline__ uint32_t wave_umax(uint32_t x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+#define HTR_DPP_MAX(ctrl) x = max(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, ctrl, 0xf, 0xf, false));
+   HTR_DPP_MAX(0x111) HTR_DPP_MAX(0x112) HTR_DPP_MAX(0x114) HTR_DPP_MAX(0x118)
+   HTR_DPP_MAX(0x142) HTR_DPP_MAX(0x143)
+#undef HTR_DPP_MAX
+#else
+   for (int o = 32; o > 0; o >>= 1) x = max(x, __shfl_xor(x, o, 64));
+#endif
+   return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+// upper word of a number >= 0: ordered as the numbers, but for equal words
+__device__ __forceinline__ uint32_t upper_word(double x) { return (uint32_t)(__double_as_longlong(x) >> 32); }
+__device__ __forceinline__ uint32_t upper_word(float x) { return (uint32_t)__float_as_int(x); }
 
 // lane t: x of lane t - 1, and x0 in lane 0
 __device__ __forceinline__ double wave_shift(double x, double x0)
@@ -692,9 +712,14 @@ struct ChemWave {
       for (int j = j0; j < j1; j++) {
          const T_ dum = vvi*fabs(row[0]);
          const bool cand = act && pos >= j && dum >= (T_)0;       // not a NaN
-         const double mine = cand ? (double)dum : -1.0;
-         const double best = wave_dmax(mine);
-         unsigned long long hit = __ballot(cand && mine == best);
+         const T_ inv = (T_)1/row[0];                             // of every row: does not wait for the pivot
+         const uint32_t key = cand ? upper_word(dum) + 1u : 0u;
+         const uint32_t top = wave_umax(key);
+         unsigned long long hit = __ballot(cand && key == top);
+         if (sizeof(T_) == 8 && (hit & (hit - 1))) {              // equal upper words: the numbers themselves
+            const double best = wave_dmax((cand && key == top) ? (double)dum : -1.0);
+            hit = __ballot(cand && key == top && (double)dum == best);
+         }
          if (!hit) hit = __ballot(act && pos == j);
          int P = __ffsll(hit) - 1;
          int imax = __builtin_amdgcn_readlane(pos, P);
@@ -705,8 +730,8 @@ struct ChemWave {
          if (lane == P) pos = j;
          else if (act && pos == j) pos = imax;
          T_ pv = rdlane(row[0], P);
-         if (pv == (T_)0) pv = (T_)1.0e-20;
-         const T_ dv = (T_)1/pv;
+         T_ dv = rdlane(inv, P);
+         if (pv == (T_)0) { pv = (T_)1.0e-20; dv = (T_)1/pv; }
          const T_ lij = row[0]*dv;
          const bool below = act && pos > j;
          const T_ w = below ? lij : (T_)0;
@@ -848,25 +873,27 @@ struct ChemWave {
 #pragma unroll
       for (int k = 0; k < N; k++) lu[k] = M[perm + k*N];
       const float ud = 1.0f/M[perm + l*N];
-      double ar[N];
-#pragma unroll
-      for (int k = 0; k < N; k++) ar[k] = ((l == k) ? d : 0.0) - Jm()[l + k*N];
+      // the matrix is read from LDS in every sweep, a few entries ahead: held in
+      // registers beside the factors it spilled.  r - (d - J) x is formed as
+      // r + (J - d) x, the same to the bit
+      const double *Jr = Jm() + l;
+      const double jd = Jr[l*N] - d;
       double xk = 0.0, prev = 0.0;
       bool done = false;
 #pragma unroll 1
       for (int it = 0; it < 9 && !done; it++) {
          double r = b;
          if (it > 0) {
-            double u[N + 8], t[N + 2];
+            double u[N + 8], a[N + 8], t[N + 2];
 #pragma unroll
-            for (int j = 0; j < 8 && j < N; j++) u[j] = rdlane(xk, j);
+            for (int j = 0; j < 8 && j < N; j++) { a[j] = Jr[j*N]; u[j] = rdlane(xk, j); }
 #pragma unroll
-            for (int j = 0; j < 2; j++) t[j] = ar[j]*u[j];
+            for (int j = 0; j < 2; j++) t[j] = ((l == j) ? jd : a[j])*u[j];
 #pragma unroll
             for (int j = 0; j < N; j++) {
-               if (j + 8 < N) u[j + 8] = rdlane(xk, j + 8);
-               if (j + 2 < N) t[j + 2] = ar[j + 2]*u[j + 2];
-               r -= t[j];
+               if (j + 8 < N) { a[j + 8] = Jr[(j + 8)*N]; u[j + 8] = rdlane(xk, j + 8); }
+               if (j + 2 < N) t[j + 2] = ((l == j + 2) ? jd : a[j + 2])*u[j + 2];
+               r += t[j];
                __builtin_amdgcn_sched_barrier(0);
             }
          }
