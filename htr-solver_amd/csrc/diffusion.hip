@@ -52,7 +52,8 @@ struct DiffCell {
 // (conduction + species enthalpy transport) returned
 template<class MX, bool SOA>
 __device__ __forceinline__ double species_face(double *Flux, const DMix &m, const FaceW &w, double m_s,
-                                               const DiffCell<MX, SOA> &P, const DiffCell<MX, SOA> &Q)
+                                               const DiffCell<MX, SOA> &P, const DiffCell<MX, SOA> &Q,
+                                               const double *tab)
 {
    constexpr int NS = MX::NS;
    const double rho_s = w(P.rho, Q.rho);
@@ -61,7 +62,7 @@ __device__ __forceinline__ double species_face(double *Flux, const DMix &m, cons
    double heatFlux = w(P.lam, Q.lam)*m_s*(P.T - Q.T);
    double ViCorr = 0.0;
    double hs[NS];
-   MX::SpeciesEnthalpies(m, hs, T_s);
+   MX::SpeciesEnthalpies(m, hs, T_s, tab);
 #pragma unroll
    for (int i = 0; i < NS; i++) {
       const double YiVi = w(P.Di[i], Q.Di[i])*m_s*(P.X[i] - Q.X[i])*MX::SpeciesW(m, i)*iMixW_s;
@@ -128,10 +129,12 @@ struct Diffusion {
    const DMix &m;
    const Geo &g;
    const P3 &p;
+   const double *tab;          // the species' polynomial coefficients in LDS
    uint32_t up[3], dn[3];      // offsets to the next and the previous cell along a direction
 
-   __device__ __forceinline__ Diffusion(const htr_fields &f_, const DMix &m_, const Geo &g_, const P3 &p_)
-      : f(f_), m(m_), g(g_), p(p_)
+   __device__ __forceinline__ Diffusion(const htr_fields &f_, const DMix &m_, const Geo &g_, const P3 &p_,
+                                        const double *tab_)
+      : f(f_), m(m_), g(g_), p(p_), tab(tab_)
    {
 #pragma unroll
       for (int d = 0; d < 3; d++) {
@@ -180,12 +183,12 @@ struct Diffusion {
       double Fp[NS], Fm[NS];
       Cell C;
       C.load(f, m, p.o + up[DIR]);
-      hp = species_face<MX, SOA>(Fp, m, F.wp, F.msp, C0, C);
+      hp = species_face<MX, SOA>(Fp, m, F.wp, F.msp, C0, C, tab);
 #pragma unroll
       for (int i = 0; i < NS; i++) HTR_PIN(Fp[i]);
       HTR_PIN(hp);
       C.load(f, m, p.o + dn[DIR]);
-      hm = species_face<MX, SOA>(Fm, m, F.wm, F.msm, C, C0);
+      hm = species_face<MX, SOA>(Fm, m, F.wm, F.msm, C, C0, tab);
       if (F.own) hm = hp;
 #pragma unroll
       for (int i = 0; i < NS; i++) {
@@ -270,14 +273,28 @@ struct Diffusion {
    }
 };
 
+// The faces of a cell lie between temperatures, so in a flow about a range
+// switch of the polynomials most waves straddle it.  Their coefficients come
+// from a copy in LDS instead of 90 gathers per direction through the address
+// unit that the fields' loads already fill, where the registers allow it (at
+// two waves per SIMD, which all three directions and the x direction have
+// anyway; y and z alone fit three waves without it and would spill with it:
+// 402 -> 601 us).  All three directions of 160^3 air about 6000 K 1318 -> 1073
+// us, 907-918 us at other temperatures with and without.
 template<class MX, int DIRS, bool SOA>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4)))
+__global__ void __launch_bounds__(256, (DIRS == 7 || DIRS == 1) ? 2 : 3)
 diffusion_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, uint32_t per)
 {
    constexpr int NS = MX::NS;
+   constexpr bool TAB = !MX::CP && SOA && (DIRS == 7 || DIRS == 1);
+   __shared__ double tab[TAB ? NS*36 : 1];
+   if constexpr (TAB) {
+      for (int k = threadIdx.x; k < NS*36; k += 256) tab[k] = mix->sp[k/36].cp[k/12 % 3][k % 12];
+      __syncthreads();
+   }
    P3 p;
    if (!strip_cell(g, per, p)) return;
-   const Diffusion<MX, DIRS, SOA> D(f, *mix, g, p);
+   const Diffusion<MX, DIRS, SOA> D(f, *mix, g, p, TAB ? tab : nullptr);
    // species first, then momentum and energy, so that the species' cell values
    // are not held beside the velocity gradients; only the faces' heat fluxes
    // pass from one to the other

@@ -179,11 +179,14 @@ HD const double *cp_range(const DSpec &s, double T)
 // them; nearly every wave has all its lanes in one range, and then the
 // coefficients come through scalar loads and enter as scalar operands.  A wave
 // that straddles a switch (and a mixture too large to hold its species'
-// ranges) gathers.  256^3 air: Roe pass 0.79 -> 0.71 ms per direction (233 ->
+// ranges) gathers, from tab where the kernel has copied the coefficients to
+// LDS ([species][range][12], see diffusion_kernel).  (Selecting between the
+// ranges' scalar coefficients, or taking the ranges one after another, was
+// slower: 40 registers more, or the scalar loads' latency twice.)  256^3 air: Roe pass 0.79 -> 0.71 ms per direction (233 ->
 // 147 VGPRs).  The chemistry source evaluates them once per cell and keeps the
 // gathers (0.78 ms; 0.87 ms this way, for a wave less per SIMD).
 template<int NS, class M, class F>
-HD void species_loop(const M &m, double T, F f)
+HD void species_loop(const M &m, double T, F f, const double *tab = nullptr)
 {
 #ifdef __HIP_DEVICE_COMPILE__
    if constexpr (NS <= 8) {
@@ -206,7 +209,8 @@ HD void species_loop(const M &m, double T, F f)
       } else {
 #pragma unroll
          for (int i = 0; i < NS; i++) {
-            f(i, m.sp[i], cp_range(m.sp[i], T));
+            const DSpec &s = m.sp[i];
+            f(i, s, tab ? tab + (i*3 + (T > s.tHi ? 0 : T > s.tLo ? 1 : 2))*12 : cp_range(s, T));
             __builtin_amdgcn_sched_barrier(0);
          }
       }
@@ -362,11 +366,11 @@ struct Mix {
       return sp_enthalpy(m.sp[i], T*m.TRef)*m.ieRef;
    }
    // all species at once (the face enthalpies of the diffusion)
-   HD static void SpeciesEnthalpies(const DMix &m, double *h, double Tn)
+   HD static void SpeciesEnthalpies(const DMix &m, double *h, double Tn, const double *tab = nullptr)
    {
       if (CP) { h[0] = m.gamma/(m.gamma - 1)*m.R*Tn; return; }
       const double T = Tn*m.TRef, Tinv = 1.0/T, logT = log(T);
-      species_loop<NS>(m, T, [&](int i, const DSpec &s, const double *c) { h[i] = poly_enthalpy(s, c, T, Tinv, logT)*m.ieRef; });
+      species_loop<NS>(m, T, [&](int i, const DSpec &s, const double *c) { h[i] = poly_enthalpy(s, c, T, Tinv, logT)*m.ieRef; }, tab);
    }
    HD static double InternalEnergy(const DMix &m, double Tn, const double *Y)
    {
