@@ -276,17 +276,18 @@ struct Diffusion {
 // The faces of a cell lie between temperatures, so in a flow about a range
 // switch of the polynomials most waves straddle it.  Their coefficients come
 // from a copy in LDS instead of 90 gathers per direction through the address
-// unit that the fields' loads already fill, where the registers allow it (at
-// two waves per SIMD, which all three directions and the x direction have
-// anyway; y and z alone fit three waves without it and would spill with it:
-// 402 -> 601 us).  All three directions of 160^3 air about 6000 K 1318 -> 1073
-// us, 907-918 us at other temperatures with and without.
+// unit that the fields' loads already fill, where the registers allow it: at
+// two waves per SIMD, which all three directions at once have anyway (160^3 air
+// about 6000 K 1318 -> 1073 us, 907-918 us at other temperatures with and
+// without).  One direction alone fits three waves without the copy and would
+// spill with it; along x, 140^3, at 2700 K and about 6000 K: 336 and 388 us, with
+// the copy at two waves 358 and 378.
 template<class MX, int DIRS, bool SOA>
-__global__ void __launch_bounds__(256, (DIRS == 7 || DIRS == 1) ? 2 : 3)
+__global__ void __launch_bounds__(256, DIRS == 7 ? 2 : 3)
 diffusion_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, uint32_t per)
 {
    constexpr int NS = MX::NS;
-   constexpr bool TAB = !MX::CP && SOA && (DIRS == 7 || DIRS == 1);
+   constexpr bool TAB = !MX::CP && SOA && DIRS == 7;
    __shared__ double tab[TAB ? NS*36 : 1];
    if constexpr (TAB) {
       for (int k = threadIdx.x; k < NS*36; k += 256) tab[k] = mix->sp[k/36].cp[k/12 % 3][k % 12];
