@@ -93,12 +93,16 @@ __device__ __forceinline__ void smooth_minus(const double *v, double *s)
 
 // 1/d to within a rounding, for quantities that only enter a stencil
 // selection (see ipow6): the hardware's estimate (2^-24) and one third-order
-// correction, 4 instructions against the 11 of a division
+// correction, 4 instructions against the 11 of a division.  INF: 1/infinity is
+// 0, for one instruction more (the plain correction forms infinity times 0);
+// the ratios tau6/(s + eps) do without it, as tau6 is then infinite or not a
+// number itself and so is no ratio.
+template<bool INF>
 __device__ __forceinline__ double sel_rcp(double d)
 {
 #ifdef __HIP_DEVICE_COMPILE__
    const double r = __builtin_amdgcn_rcp(d);
-   const double e = fma(-d, r, 1.0);
+   const double e = fma(-(INF ? fmin(d, 1.7976931348623157e308) : d), r, 1.0);
    return fma(r, fma(e, e, e), r);
 #else
    return 1.0/d;
@@ -165,7 +169,7 @@ __device__ __forceinline__ double teno_reconstruct(const double *v, int t, uint3
    const double tau6 = fabs(s[3] - (s[2] + s[1] + 4*s[0])*(1.0/6.0));
    double chi[4], a[4];
 #pragma unroll
-   for (int k = 0; k < 4; k++) { chi[k] = tau6*sel_rcp(s[k] + eps); a[k] = ipow6(1 + chi[k]); }
+   for (int k = 0; k < 4; k++) { chi[k] = tau6*sel_rcp<false>(s[k] + eps); a[k] = ipow6(1 + chi[k]); }
    if (!STD && (OP != 1 || t != Std_node)) {
 #pragma unroll
       for (int k = 0; k < 4; k++) if (Coeffs[k] < 1e-10) a[k] = 0.0;
@@ -185,7 +189,7 @@ __device__ __forceinline__ double teno_reconstruct(const double *v, int t, uint3
          double eta = 0.0;
 #pragma unroll
          for (int k = 0; k < 4; k++) {
-            const double r = (2*var[k]*var[k+1] + Ren_eps)*sel_rcp(sq[k] + sq[k+1] + Ren_eps);
+            const double r = (2*var[k]*var[k+1] + Ren_eps)*sel_rcp<true>(sq[k] + sq[k+1] + Ren_eps);
             eta = k ? dmin(eta, r) : r;
          }
          const double delta = 1 - dmin(eta*Ren_irc, 1.0);
@@ -198,7 +202,7 @@ __device__ __forceinline__ double teno_reconstruct(const double *v, int t, uint3
    } else {
       const double Smooth_pow = 12.5, Shock_pow = 3.0, iH = 1e-1, Diff_pow = Smooth_pow - Shock_pow;
       const double chiMax = dmax(chi[0], dmax(chi[1], dmax(chi[2], chi[3])));
-      const double theta = sel_rcp(1 + chiMax*iH);
+      const double theta = sel_rcp<true>(1 + chiMax*iH);
       const int power = min(max((int)floor(Shock_pow + Diff_pow*theta), 0), 13);
       cut = (double)c_st.p10[power];
    }
