@@ -42,7 +42,8 @@ static std::map<std::pair<int, uintptr_t>, Workspace*> g_ws;   // (device, strea
 static bool g_ready[16];
 
 // grows a workspace buffer; the old buffer is freed only after the stream's
-// earlier work (the only work that can use it) has finished.  Called with
+// earlier work has finished, which is all that can use it (side streams use a
+// caller stream's buffers, but that stream follows them: SideWork).  Called with
 // the workspace's own lock held, not the library's: a growth on one stream
 // does not stall calls on others.
 static int grow(hipStream_t s, void **p, int64_t &cap, int64_t need, size_t elem, const char *what)
@@ -487,10 +488,10 @@ static int need(const htr_view &v, const char *name)
 }
 
 // Side streams of the full RHS with overlap, per (device, caller stream):
-// one stream per direction for that direction's TENO passes (each stream has
-// its own workspace, so the three face buffers live at once) and the events
-// of the hand-overs.  Default priority, non-blocking (ordered by the events
-// only).
+// one stream per direction for that direction's TENO passes, each with its own
+// face list and records; the total enthalpy they read and the face fluxes they
+// write are in the caller stream's workspace.  Default priority, non-blocking
+// (ordered by the events only).
 struct RhsAux {
    hipStream_t ts[3] = {};
    hipEvent_t  h = nullptr;           // caller stream: total enthalpy formed
@@ -519,6 +520,30 @@ static RhsAux *rhs_aux(hipStream_t s)
    return a;
 }
 
+// The side streams that received work of a call.  They use the caller stream's
+// buffers, so that stream has to follow them on every way out of the call, also
+// where a later step fails: a buffer is rewritten or freed after that stream's
+// own earlier work (grow).
+struct SideWork {
+   RhsAux &aux;
+   hipStream_t s;
+   bool pending[3] = {};
+   bool join()
+   {
+      bool ok = true;
+      for (int d = 2; d >= 0; d--) {
+         if (!pending[d]) continue;
+         pending[d] = false;
+         if (hipEventRecord(aux.teno[d], aux.ts[d]) != hipSuccess || hipStreamWaitEvent(s, aux.teno[d], 0) != hipSuccess) {
+            (void)hipStreamSynchronize(aux.ts[d]);
+            ok = false;
+         }
+      }
+      return ok;
+   }
+   ~SideWork() { join(); }
+};
+
 // The hybrid Euler sweeps with each direction's TENO passes on a side stream:
 // total enthalpy (caller stream), then the TENO passes of z, y, x on their
 // side streams, overlapping the chemistry source on the caller stream; the KG
@@ -534,17 +559,16 @@ static int euler_overlapped(const htr_fields &fr, const htr_mix *m, const Geo &g
    int rc = enthalpy_launch<MX>(fr, geo, s);
    if (rc) return rc;
    if (hipEventRecord(aux->h, s) != hipSuccess) return set_error(HTR_E_DEVICE, "event record failed");
+   SideWork side{*aux, s};
    for (int d = 2; d >= 0; d--) {
-      if (hipStreamWaitEvent(aux->ts[d], aux->h, 0) != hipSuccess)
-         return set_error(HTR_E_DEVICE, "stream wait failed");
+      if (hipStreamWaitEvent(aux->ts[d], aux->h, 0) != hipSuccess) return set_error(HTR_E_DEVICE, "stream wait failed");
+      side.pending[d] = true;
       if ((rc = rhs_euler_part<MX>(d, 0, HTR_EULER_HYBRID, fr, m->dev, geo, RK0, RK1, dt, dec, aux->ts[d], s))) return rc;
-      if (hipEventRecord(aux->teno[d], aux->ts[d]) != hipSuccess) return set_error(HTR_E_DEVICE, "event record failed");
    }
    if (chem_source && !m->host.constprop) rc = chem_source_launch<MixAir>(fr, m->dev, geo, s, true);
    else                                   rc = zero_rhs_launch(fr, geo, m->host.nSpec + 4, s);
    if (rc) return rc;
-   for (int d = 2; d >= 0; d--)
-      if (hipStreamWaitEvent(s, aux->teno[d], 0) != hipSuccess) return set_error(HTR_E_DEVICE, "stream wait failed");
+   if (!side.join()) return set_error(HTR_E_DEVICE, "stream wait failed");
    return rhs_euler_part<MX>(0, 1, HTR_EULER_HYBRID, fr, m->dev, geo, RK0, RK1, dt, dec, s, s);
 }
 

@@ -1,0 +1,64 @@
+"""Child process of tests/test_emu_faults.py: library calls that fail on the
+way (tests/emu_faults/hip), through the kernel source compiled for the CPU.
+Prints "CASE <name> <figures>"; exits non-zero on the first that is wrong."""
+import ctypes as C
+import os
+import sys
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path[:0] = [os.path.join(os.path.dirname(HERE), "emu")]
+
+import run_emu as R  # noqa: E402
+from hotpath import complete_state, gpu_mix, tgv_state  # noqa: E402
+
+H = R.H
+H.init(0)
+LIB = H.lib()
+for _name, _res, _arg in (("arm", None, C.c_long), ("calls", C.c_long, None), ("launches", C.c_long, None),
+                          ("limit", None, C.c_size_t), ("unfollowed", C.c_int, C.c_void_p)):
+    _f = getattr(LIB, "hipfault_" + _name)
+    _f.restype, _f.argtypes = _res, [_arg] if _arg else []
+
+
+def check(ok, name, *figures):
+    print("CASE", name, *figures, flush=True)
+    if not ok:
+        sys.exit(3)
+
+
+def small_vortex(n=(6, 5, 4)):
+    st, meta = tgv_state(6)
+    st = {k: v[..., :n[2], :n[1], :n[0]].copy() for k, v in st.items()}
+    st, _ = complete_state(st, meta, n)
+    for d in range(3):
+        st["shockSensor%d" % d][:] = 0            # every face takes the TENO branch
+    return R.to_host_fs(st, 1, n), gpu_mix(meta)
+
+
+def side_streams():
+    """Whatever call or launch of a right-hand side on side streams fails: the
+    caller's stream follows all the work that was launched."""
+    H.rhs_overlap(True)
+    failed = 0
+    for k in range(1, 200):
+        fs, mix = small_vortex()
+        LIB.hipfault_arm(k)
+        try:
+            H.full_rhs(fs, 0, (1.0, 0.0), 1e-3, False, mix)
+            error = None
+        except Exception as e:
+            error = str(e)
+        calls = LIB.hipfault_calls()
+        LIB.hipfault_arm(0)
+        left = LIB.hipfault_unfollowed(None)
+        if left:
+            check(False, "side_streams", k, "left", left, error)
+        if calls < k:
+            break
+        failed += error is not None
+    check(failed >= 20 and error is None, "side_streams", k, failed)
+
+
+if __name__ == "__main__":
+    for which in sys.argv[1:]:
+        globals()[which]()
