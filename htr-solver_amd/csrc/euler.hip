@@ -696,34 +696,19 @@ euler_kg_kernel(const htr_fields f, const Geo g, const htr_view hv, const KGFace
    for (int i = 0; i < MX::NEQ; i++) *ptr_o<double, SOA>(f.Conserved_t, p.o, i) = ct[i];
 }
 
-// Pass 2: TENO-family faces, either all faces or the compacted list, in
-// three kernels that each keep a small register footprint:
+// Pass 2: TENO-family faces, either all faces or the compacted list:
 //   2a  lane per face: Roe state + eigenvalue maxima -> record
-//   2b  a wave per (component, 64 faces), face data staged in LDS: split
-//       fluxes, TENO +/- -> component, bits
-//   2c  lane per face: back-projection, limiter -> face flux, decision word
-// Buffers (capacity cap = number of faces): record NREC*cap doubles, then
-// components NEQ*cap doubles, then bits NEQ*cap bytes.
+//   2b  a block per 64 faces, face data staged in LDS: split fluxes, TENO +/-,
+//       back-projection, limiter test -> face flux, decision word
+//   2c  lane per listed face: limiter blend
+// Records: NREC*cap doubles, component-major (capacity cap = number of faces).
 struct TenoBufs {
-   double *rec, *Fc;
-   uint8_t *bits;
+   double *rec;
    int64_t cap;
 };
 
 template<class MX>
-__host__ __device__ inline int64_t teno_doubles(int64_t cap)
-{ return (Euler<MX, 0>::NREC + MX::NEQ)*cap + (MX::NEQ*cap + 7)/8; }
-
-template<class MX>
-inline TenoBufs teno_bufs(double *base, int64_t cap)
-{
-   TenoBufs b;
-   b.rec = base;
-   b.Fc = base + Euler<MX, 0>::NREC*cap;
-   b.bits = reinterpret_cast<uint8_t*>(b.Fc + MX::NEQ*cap);
-   b.cap = cap;
-   return b;
-}
+__host__ __device__ inline int64_t teno_doubles(int64_t cap) { return Euler<MX, 0>::NREC*cap; }
 
 template<class MX, int DIR, bool LISTED>
 __global__ void __launch_bounds__(256)
@@ -740,7 +725,7 @@ euler_roe_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, 
    }
 }
 
-// Passes 2b + 2c in one kernel.  A block of four waves takes chunks of 64
+// Pass 2b.  A block of four waves takes chunks of 64
 // listed TENO faces, a lane per face, in three steps between barriers:
 //   stage       the six stencil points, dealt to the waves: the point's
 //               values (conserved vector, u_n, p) are gathered and left in
@@ -1013,7 +998,7 @@ static int launch_teno(const htr_fields &f, const DMix *mix, const Geo &g, const
                        hipStream_t s)
 {
    constexpr int kMaxBlocks = 256*16;
-   const TenoBufs b = teno_bufs<MX>(w.teno, nfaces);
+   const TenoBufs b{ w.teno, nfaces };
    const unsigned nb = (unsigned)std::min<int64_t>(grid_for(nfaces, 256), kMaxBlocks);
    HTR_LAUNCH(HTR_DIR_NAME("euler_roe", DIR), (euler_roe_kernel<MX, DIR, LISTED>), dim3(nb), dim3(256), 0, s,
                       f, mix, g, hv, b, nfaces, w.list, w.counter);

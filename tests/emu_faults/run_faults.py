@@ -59,6 +59,34 @@ def side_streams():
     check(failed >= 20 and error is None, "side_streams", k, failed)
 
 
+def air_box(n=(6, 5, 4)):
+    from emu_edges_state import state
+    st, meta = state(n, 2)
+    st, _ = complete_state(st, meta, n)
+    for d in range(3):
+        st["shockSensor%d" % d][:] = 0
+    return R.to_host_fs(st, 5, n), gpu_mix(meta)
+
+
+def faces(n):
+    """faces of the largest direction of a box"""
+    return max(n[0] * n[1] * n[2] // n[d] * (n[d] + 1) for d in range(3))
+
+
+def teno_memory():
+    """A pure TENO sweep takes 22 doubles a face beside its fluxes (9 doubles a
+    face) and nothing larger."""
+    n = (15, 14, 15)               # (more than the fixed part of a workspace)
+    fs, mix = air_box(n)
+    LIB.hipfault_limit(22 * 8 * faces(n))
+    try:
+        H.update_using_teno_euler_flux(fs, 1, "TENO", (1.0, 0.0), 1e-4, mix)
+        error = None
+    except Exception as e:
+        error = str(e)
+    check(error is None, "teno_memory", error)
+
+
 if __name__ == "__main__":
     for which in sys.argv[1:]:
         globals()[which]()
