@@ -55,8 +55,11 @@ static int grow(hipStream_t s, void **p, int64_t &cap, int64_t need, size_t elem
    }
    *p = nullptr;
    cap = 0;
-   if (hipMalloc(p, elem*(size_t)need) != hipSuccess)
+   if (hipMalloc(p, elem*(size_t)need) != hipSuccess) {
+      *p = nullptr;
+      (void)hipGetLastError();         // not the next launch's
       return set_error(HTR_E_DEVICE, "%s allocation (%lld elements) failed", what, (long long)need);
+   }
    cap = need;
    return HTR_OK;
 }
@@ -68,6 +71,16 @@ int workspace_faces(Workspace &w, int64_t ndoubles, int64_t nlist, int64_t nteno
    if (!rc) rc = grow(w.stream, (void**)&w.list, w.list_cap, nlist, sizeof(int32_t), "face list");
    if (!rc) rc = grow(w.stream, (void**)&w.teno, w.teno_cap, nteno, sizeof(double), "TENO face buffer");
    return rc;
+}
+
+bool workspace_faces_fit(Workspace &w, int64_t ndoubles, bool again)
+{
+   std::lock_guard<std::mutex> lk(w.mu);
+   if (w.faces_refused && ndoubles >= w.faces_refused && !again) return false;
+   const bool ok = grow(w.stream, (void**)&w.faces, w.faces_cap, ndoubles, sizeof(double), "face buffer") == HTR_OK;
+   if (!ok) w.faces_refused = ndoubles;
+   else if (ndoubles >= w.faces_refused) w.faces_refused = 0;
+   return ok;
 }
 
 int workspace_enthalpy(Workspace &w, int64_t ndoubles)
@@ -1036,7 +1049,8 @@ int htr_workspace_reserve(const htr_grid *g, const htr_fields *f, const htr_mix 
    }
    Workspace *w = workspace((hipStream_t)stream);
    if (!w) return HTR_E_DEVICE;
-   if ((rc = workspace_faces(*w, need.faces, need.list, need.teno))) return rc;
+   const bool fit = workspace_faces_fit(*w, need.faces, true);
+   if ((rc = workspace_faces(*w, fit ? 0 : need.faces_one, need.list, need.teno))) return rc;
    if ((rc = workspace_enthalpy(*w, need.hbuf))) return rc;
    if (g_overlap) {
       // the side streams of the full RHS, one direction's TENO faces each
@@ -1089,7 +1103,9 @@ static int full_rhs(const htr_grid *g, const htr_fields *f, int scheme, double R
    // total enthalpy once for the three sweeps
    rc = (k == K_CP) ? enthalpy_launch<MixCP>(fr, geo, s) : enthalpy_launch<MixAir>(fr, geo, s);
    if (rc) return rc;
-   if (scheme == HTR_EULER_HYBRID || scheme == HTR_EULER_KG) {
+   const bool at_once = scheme == HTR_EULER_KG ||
+      (scheme == HTR_EULER_HYBRID && (k == K_CP ? rhs_faces_fit<MixCP>(geo, s) : rhs_faces_fit<MixAir>(geo, s)));
+   if (at_once) {
       for (int d = (scheme == HTR_EULER_KG) ? -1 : 2; d >= -1; d--) {
          const int part = d < 0 ? 1 : 0;
          rc = (k == K_CP) ? rhs_euler_part<MixCP>(d, part, scheme, fr, m->dev, geo, RK0, RK1, dt, dec, s, s)

@@ -1164,6 +1164,18 @@ int rhs_euler_part(int dir, int part, int scheme, const htr_fields &f, const DMi
    return kg_cells<MX, 7, false>(f, g, hv, F, dec, s);
 }
 
+template<class MX>
+bool rhs_faces_fit(const Geo &g, hipStream_t s)
+{
+   for (int64_t n : { Faces<0>::count(g), Faces<1>::count(g), Faces<2>::count(g) })
+      if (n*MX::NEQ >= (1ll << 31)) return true;      // refused by the sweeps
+   Workspace *w = workspace(s);
+   return !w || workspace_faces_fit(*w, rhs_face_base<MX>(g, -1));
+}
+
+template bool rhs_faces_fit<MixCP>(const Geo &, hipStream_t);
+template bool rhs_faces_fit<MixAir>(const Geo &, hipStream_t);
+
 template int rhs_euler_part<MixCP>(int, int, int, const htr_fields &, const DMix *, const Geo &, double, double,
                                    const DtArg &, const htr_view &, hipStream_t, hipStream_t);
 template int rhs_euler_part<MixAir>(int, int, int, const htr_fields &, const DMix *, const Geo &, double, double,
@@ -1191,14 +1203,15 @@ int enthalpy_launch(const htr_fields &f, const Geo &g, hipStream_t s)
 template int enthalpy_launch<MixCP>(const htr_fields &, const Geo &, hipStream_t);
 template int enthalpy_launch<MixAir>(const htr_fields &, const Geo &, hipStream_t);
 
-// Workspace sizes of the Euler sweeps (every scheme, every direction) and
-// of the diffusion sweeps (heat flux per face) over the rect of g.
+// Workspace sizes of the Euler sweeps (every scheme, every direction) over the
+// rect of g.
 template<class MX>
 WorkspaceNeed euler_workspace_need(const Geo &g)
 {
    WorkspaceNeed n;
    auto dir = [&](int64_t nfaces) {
       n.faces += nfaces*MX::NEQ;               // the full right-hand side holds all three
+      n.faces_one = std::max(n.faces_one, nfaces*MX::NEQ);
       n.list = std::max(n.list, 2*nfaces);
       n.teno = std::max(n.teno, teno_doubles<MX>(nfaces));
    };

@@ -23,11 +23,12 @@ struct Workspace {
    double  *partial = nullptr;      // per-block partial maxima, capacity kPartial
    double  *result_host = nullptr;  // pinned, 1 double
    int     *counter = nullptr;      // device ints: [0] failure counter, [1] face-list length
-   double  *faces = nullptr;        // face fluxes of one sweep, capacity faces_cap doubles
+   double  *faces = nullptr;        // face fluxes, of one sweep or of a right-hand side's three; capacity faces_cap doubles
    int32_t *list = nullptr;         // compacted face indices, capacity list_cap
    double  *teno = nullptr;         // TENO face records, capacity teno_cap doubles
    double  *hbuf = nullptr;         // per-cell total enthalpy of the Euler sweeps, capacity hbuf_cap doubles
    int64_t  faces_cap = 0, list_cap = 0, teno_cap = 0, hbuf_cap = 0;
+   int64_t  faces_refused = 0;      // face fluxes that there was no memory for, 0: none (workspace_faces_fit)
    std::mutex mu;                   // guards growth of this workspace's buffers
    static constexpr int64_t kPartial = 1 << 16;
 };
@@ -36,8 +37,13 @@ Workspace *workspace(hipStream_t s);   // null on allocation failure (error set)
 // needs more than any earlier call on this stream, or than a reservation)
 int workspace_faces(Workspace &w, int64_t ndoubles, int64_t nlist, int64_t nteno);
 int workspace_enthalpy(Workspace &w, int64_t ndoubles);
-// buffer sizes a rect needs (maximum over directions and schemes)
-struct WorkspaceNeed { int64_t faces = 0, list = 0, teno = 0, hbuf = 0; };
+// the same for face fluxes that a caller can do without: false if there is no
+// memory for them.  Not tried again for as many or more, but by a reservation
+// (again)
+bool workspace_faces_fit(Workspace &w, int64_t ndoubles, bool again = false);
+// buffer sizes a rect needs: face fluxes of a right-hand side's three sweeps and
+// of one, the others the maximum over directions and schemes
+struct WorkspaceNeed { int64_t faces = 0, faces_one = 0, list = 0, teno = 0, hbuf = 0; };
 template<class MX> WorkspaceNeed euler_workspace_need(const Geo &g);
 template<class MX> int enthalpy_launch(const htr_fields &f, const Geo &g, hipStream_t s);
 
@@ -53,6 +59,9 @@ template<class MX> int euler_dispatch(int dir, int scheme, const htr_fields &f, 
 template<class MX> int rhs_euler_part(int dir, int part, int scheme, const htr_fields &f, const DMix *mix,
                                       const Geo &g, double RK0, double RK1, const DtArg &dt, const htr_view &dec,
                                       hipStream_t ts, hipStream_t s);
+// false where there is no memory for the face fluxes of all three sweeps at
+// once: they are then taken one by one (euler_dispatch), equal to the bit
+template<class MX> bool rhs_faces_fit(const Geo &g, hipStream_t s);
 // dirs: one direction (1 x, 2 y, 4 z) or 7, all three in the order z, y, x
 template<class MX> int diffusion_dispatch(int dirs, const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s);
 template<class MX> int properties_launch(const htr_fields &f, const DMix *mix, const Geo &g, hipStream_t s);

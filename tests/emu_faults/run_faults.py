@@ -87,6 +87,31 @@ def teno_memory():
     check(error is None, "teno_memory", error)
 
 
+def rhs_memory():
+    """A full right-hand side where there is memory for one direction's face
+    fluxes (9 doubles a face) but not for three: the same result to the bit, and
+    not a call more that is refused; the larger buffer is tried for again by a
+    reservation alone."""
+    n = (15, 14, 15)
+    out = []
+    for limit in (0, 22 * 8 * faces(n)):
+        fs, mix = air_box(n)
+        LIB.hipfault_limit(limit)
+        if limit:
+            # (a workspace that has grown keeps what it has: another stream's)
+            R.A.stream_ptr = lambda stream=None: C.c_void_p(8)
+        for call in range(2):
+            try:
+                H.full_rhs(fs, 0, (1.0, 0.0), 1e-4, True, mix)
+                H.workspace_reserve(fs, mix)
+                error = None
+            except Exception as e:
+                error = str(e)
+            check(error is None, "rhs_memory", limit, call, error)
+            out.append(fs["Conserved_t"].numpy().copy())
+    check(all((o == out[0]).all() for o in out), "rhs_memory equal")
+
+
 if __name__ == "__main__":
     for which in sys.argv[1:]:
         globals()[which]()
