@@ -104,13 +104,6 @@ class Mixture:
             pass
 
 
-# the views of htr_fields in the order of the struct, without the profiles that end it
-FIELD_ORDER = tuple("%s%d" % (k, d) for k in ("nType", "m_e", "m_d", "m_s") for d in range(3)) + (
-    "rho", "mu", "lam", "Di", "SoS", "pressure", "temperature", "MassFracs", "MolarFracs", "velocity", "Conserved",
-    "Conserved_old", "Conserved_t", "Conserved_t_old", "shockSensor0", "shockSensor1", "shockSensor2", "DucrosSensor")
-_PACK_FIELDS = struct.Struct("=" + "qqqqq" * len(FIELD_ORDER)).pack_into
-
-
 def make_grid(n, lo=(0, 0, 0), hi=None, bounds_lo=(0, 0, 0)):
     """Grid over a box of n = (nx, ny, nz) cells whose first cell has absolute
     coordinates bounds_lo; exec rect [lo, hi] in box-relative indices."""
@@ -129,6 +122,24 @@ VECTORS = {"Di": "ns", "MassFracs": "ns", "MolarFracs": "ns", "velocity": 3,
            "Conserved": "neq", "Conserved_old": "neq", "Conserved_t": "neq", "Conserved_t_old": "neq"}
 PROFILES = {"MolarFracs_profile": "ns", "velocity_profile": 3, "temperature_profile": 0,
             "dudtBoundary": 3, "dTdtBoundary": 0}
+
+
+def field_order(fields):
+    """Names of a FieldSet's tensors in the order of the views of the struct (the
+    members of an array of views numbered), without the profiles that end it."""
+    names = []
+    for k, t in fields._fields_:
+        if k in PROFILES:
+            break
+        names += [k] if t is View else ["%s%d" % (k, d) for d in range(t._length_)]
+    size = C.sizeof(View)
+    if size != 40 or C.sizeof(fields) != size * (len(names) + len(PROFILES)):
+        raise TypeError("%s is not a run of views that ends with the profiles" % fields.__name__)
+    return tuple(names)
+
+
+FIELD_ORDER = field_order(Fields)
+_PACK_FIELDS = struct.Struct("=" + "qqqqq" * len(FIELD_ORDER)).pack_into
 
 
 class FieldSet:
