@@ -331,8 +331,12 @@ static int upload(htr_mix *m)
    if (!m->dev && hipMalloc((void **)&m->dev, at + bytes) != hipSuccess)
       return set_error(HTR_E_DEVICE, "mixture allocation failed");
    if (hipMemcpy(m->dev, &m->host, sizeof(DMix), hipMemcpyHostToDevice) != hipSuccess ||
-       (bytes && hipMemcpy(reinterpret_cast<char*>(m->dev) + at, rows.data(), bytes, hipMemcpyHostToDevice) != hipSuccess))
+       (bytes && hipMemcpy(reinterpret_cast<char*>(m->dev) + at, rows.data(), bytes, hipMemcpyHostToDevice) != hipSuccess)) {
+      // before it is finalized a mixture can still get reactions: the next
+      // upload allocates for them
+      if (!m->finalized) { (void)hipFree(m->dev); m->dev = nullptr; }
       return set_error(HTR_E_DEVICE, "mixture upload failed");
+   }
    m->finalized = 1;
    return HTR_OK;
 }

@@ -112,6 +112,33 @@ def rhs_memory():
     check(all((o == out[0]).all() for o in out), "rhs_memory equal")
 
 
+def mixture_upload():
+    """A finalize that fails after its allocation, then more reactions, then one
+    that does not fail: the image has room for them all."""
+    from htr_amd import cases, mechanism
+    mech = mechanism.synthetic_30(0)
+    few = dict(mech, reactions=mech["reactions"][:1])
+    check_, codes = R.A.check, []
+    for k in (2, 3):                               # the copy of the mixture, the copy of its rows
+        R.A.check = codes.append
+        LIB.hipfault_arm(k)
+        mix = H.Mixture.from_mechanism(few)
+        LIB.hipfault_arm(0)
+        r = mech["reactions"][0]
+        two = lambda key, t: ((C.c_int * 2)(*[e[0] for e in r[key]]), (t * 2)(*[e[1] for e in r[key]]))
+        ei, en = two("educts", C.c_float)
+        pi, pn = two("products", C.c_float)
+        for _ in range(179):
+            codes.append(LIB.htr_mix_add_reaction(mix.h, r["kind"], r["A"], r["n"], r["EovR"], 1, 2, ei, en, 2, pi, pn,
+                                                  0, None, None))
+        xr = (C.c_double * 30)(*mech["XiRef"])
+        codes.append(LIB.htr_mix_finalize(mix.h, mech["PRef"], mech["TRef"], mech["LRef"], xr))
+        R.A.check = check_
+        failed = [c for c in codes if c]
+        check(len(failed) == 1, "mixture_upload", k, failed)
+        codes.clear()
+
+
 if __name__ == "__main__":
     for which in sys.argv[1:]:
         globals()[which]()

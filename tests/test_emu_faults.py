@@ -27,7 +27,7 @@ def fault_lib(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("which", ["side_streams", "teno_memory", "rhs_memory"])
+@pytest.mark.parametrize("which", ["side_streams", "teno_memory", "rhs_memory", "mixture_upload"])
 def test_failed_calls(fault_lib, which):
     asan = subprocess.run(["gcc", "-print-file-name=libasan.so"], capture_output=True, text=True).stdout.strip()
     env = dict(os.environ, HTR_AMD_LIBRARY=fault_lib, LD_PRELOAD=asan, ASAN_OPTIONS="detect_leaks=0",
