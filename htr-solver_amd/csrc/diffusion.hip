@@ -366,21 +366,23 @@ diffusion_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, 
 // the thread before: every face is formed once and every cell loaded once, but
 // for the block's first and last cells, which only hand on (blocks overlap by
 // two).  Everything is handed on through LDS, and the cell's own values are read
-// back from there too, so that 74 registers suffice and four blocks share a CU
-// (values in registers: 136, three blocks, 140^3 along y and z 10 % slower).
-// Per-point arrays keep them in registers, three blocks per CU: with four the
-// vector cache loses the records that a thread reads component by component
-// (139x67x101 along x 178, now 158 us).
+// back from there too, so that 120 registers suffice and four blocks share a CU
+// (values in registers: three blocks, 140^3 along y and z 10 % slower).  All loads
+// go out before the first barrier; loaded where they are used, some after three
+// barriers, a 200^2 box of one species took 8.8-9.0 us, now 7.5, and 140^3 air
+// 5 to 12 % more.  Per-point arrays share a CU three blocks at a time: with four,
+// or with two, the vector cache loses the records that a thread reads component by
+// component (139x67x101 along x 124 us, two blocks 138).
 // Bound by memory: 140^3 air has 0.98 GB that the pass cannot do without.  Its
 // time with the clearing of Conserved_t before it, along x, y and z; in brackets
 // with a thread per cell that forms both its faces, then with the walks along
 // lines before that, which formed each face once but passed twice over the cells:
-//   140^3, 2700 K                     264 295 285  (320 314 312; 333 385 369) us
+//   140^3, 2700 K                     251 280 260  (320 314 312; 333 385 369) us
 //   140^3, 6000 K, where waves straddle
-//     a range of the polynomials      280 318 304  (384 388 393; 331 384 371)
-//   139x67x101, 6000 K                 98 104 104  (143 142 142; 117 126 124)
-//   the same as per-point arrays      159 157 161  (229 229 227; 179 170 167)
-//   700x500, 2700 K                    37  40      ( 43  43; 49 78)
+//     a range of the polynomials      260 296 269  (384 388 393; 331 384 371)
+//   139x67x101, 6000 K                 93 103  98  (143 142 142; 117 126 124)
+//   the same as per-point arrays      135 136 134  (229 229 227; 179 170 167)
+//   700x500, 2700 K                    36  42      ( 43  43; 49 78)
 template<int DIR> struct Lines {
    static constexpr int LINES = (DIR == 0) ? 1 : 16, CELLS = 256/LINES, MINE = CELLS - 2;
    static constexpr int B = (DIR == 2) ? 1 : 2;      // the other cross direction of y and z
@@ -458,8 +460,8 @@ template<class MX, int DIR, bool SOA>
 __global__ void __launch_bounds__(256, 3)
 diffusion_line_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, uint32_t per)
 {
-   constexpr int NS = MX::NS, NV = 3*NS + 4;
-   // per-point arrays: LDS for three blocks per CU, not more
+   constexpr int NS = MX::NS, NV = LdsCell<MX>::N;
+   // per-point arrays of several species: LDS for three blocks per CU, not more
    constexpr int COLS = (!SOA && NV < 26 && NS > 1) ? 26 : (NV > 8) ? NV : 8;
    __shared__ double buf[COLS*256];
    P3 p;
@@ -470,51 +472,50 @@ diffusion_line_kernel(const htr_fields f, const DMix *__restrict__ mix, const Ge
    const Diffusion<MX, SOA> D(f, *mix, g, p, nullptr);
    const int t = ldo<int, SOA>(f.nType[DIR], p.o);
    const bool own = i == 0 && left_node(t);          // as in Diffusion::faces
-   double hp, hm;
-   {
-      double Fp[NS + 1], Fm[NS + 1];
-      DiffCell<MX, SOA> C;
-      C.load(f, *mix, p.o);
-      if constexpr (SOA) {
-         LdsCell<MX>::put(buf + me, C);
-         __syncthreads();
-         const LdsCell<MX> P(buf + me), Q(buf + next);
-         Fp[NS] = species_face<MX>(Fp, *mix, D.weights(t), ldo<double, SOA>(f.m_s[DIR], p.o), P, Q, nullptr);
-      } else {
-         DiffCell<MX, SOA> Q;
-         static_assert(sizeof(Q) == NV*sizeof(double), "a cell's values, one after the other");
-         hand_on<NV>(buf, next, &C.X[0], &Q.X[0]);
-         Fp[NS] = species_face<MX>(Fp, *mix, D.weights(t), ldo<double, SOA>(f.m_s[DIR], p.o), C, Q, nullptr);
-      }
-      hand_on<NS + 1>(buf, prev, Fp, Fm);
-      hp = Fp[NS];
-      hm = own ? hp : Fm[NS];
-      const double md = ldo<double, SOA>(f.m_d[DIR], p.o);
-#pragma unroll
-      for (int k = 0; k < NS; k++) {
-         if (own) Fm[k] = Fp[k];
-         if (mine) *ptr_o<double, SOA>(f.Conserved_t, p.o, k) += (Fp[k] - Fm[k])*md;
-      }
-   }
-   // velocity, viscosity and transverse gradients of the cell and of the next
-   double v0[8], v1[8], Fp[4], Fm[4];
+   // everything that is loaded, before the first barrier: velocity, viscosity and
+   // transverse gradients are for the second part
+   const double ms = ldo<double, SOA>(f.m_s[DIR], p.o), md = ldo<double, SOA>(f.m_d[DIR], p.o);
+   DiffCell<MX, SOA> C;
+   C.load(f, *mix, p.o);
+   double v0[8], ct[NS + 4];
 #pragma unroll
    for (int k = 0; k < 3; k++) v0[k] = D.vel(p.o, k);
    v0[3] = ldo<double, SOA>(f.mu, p.o);
    const Transverse<DIR> G0 = D.template transverse<DIR>(p.o, v0);
    v0[4] = G0.a1; v0[5] = G0.b1; v0[6] = G0.a2; v0[7] = G0.b2;
+#pragma unroll
+   for (int k = 0; k < NS + 4; k++) ct[k] = ldo<double, SOA>(f.Conserved_t, p.o, k);
+   double hp, hm;
+   {
+      double Fp[NS + 1], Fm[NS + 1];
+      LdsCell<MX>::put(buf + me, C);
+      __syncthreads();
+      const LdsCell<MX> P(buf + me), Q(buf + next);
+      Fp[NS] = species_face<MX>(Fp, *mix, D.weights(t), ms, P, Q, nullptr);
+      hand_on<NS + 1>(buf, prev, Fp, Fm);
+      hp = Fp[NS];
+      hm = own ? hp : Fm[NS];
+#pragma unroll
+      for (int k = 0; k < NS; k++) {
+         if (own) Fm[k] = Fp[k];
+         ct[k] += (Fp[k] - Fm[k])*md;
+      }
+   }
+   double v1[8], Fp[4], Fm[4];
    hand_on<8>(buf, next, v0, v1);
    const Transverse<DIR> G1 = { v1[4], v1[5], v1[6], v1[7] };
    const FaceW w = D.weights(t);
-   const double ms = ldo<double, SOA>(f.m_s[DIR], p.o), md = ldo<double, SOA>(f.m_d[DIR], p.o);
    // the plus face of an own cell takes its left gradients at the next cell
    // (Diffusion::stress), its minus face the cell's own
    Fp[3] = stress_face<DIR>(Fp, w, ms, v0, v1, v0[3], v1[3], own ? G1 : G0, G1) - hp;
    hand_on<4>(buf, prev, Fp, Fm);
    if (own) Fm[3] = stress_face<DIR>(Fm, w, ms, v0, v1, v0[3], v1[3], G0, G1) - hm;
 #pragma unroll
-   for (int k = 0; k < 4; k++)
-      if (mine) *ptr_o<double, SOA>(f.Conserved_t, p.o, NS + k) += (Fp[k] - Fm[k])*md;
+   for (int k = 0; k < 4; k++) ct[NS + k] += (Fp[k] - Fm[k])*md;
+   if (mine) {
+#pragma unroll
+      for (int k = 0; k < NS + 4; k++) *ptr_o<double, SOA>(f.Conserved_t, p.o, k) = ct[k];
+   }
 }
 
 template<class MX, bool SOA>
