@@ -58,11 +58,10 @@ RHS_BYTES_PER_CELL = 495.0
 #   enthalpy        per cell: rhoE, p, rho read, H written = 32 B
 KERNEL_BYTES = {"euler_classify": 5.0, "euler_kg": 271.0, "euler_roe": 272.0, "euler_teno": 416.0,
                 "euler_divergence": 224.0, "diffusion": 380.0, "chem_source_kernel": 136.0, "enthalpy": 32.0}
-# FP64 operations per unit of the compute-bound kernels (hand count of the
-# source, FMA-free build: per component the species sums and split fluxes of
-# six points ~600, two TENO reconstructions ~300; nine components plus the
-# back-projection and limiter test ~150)
-KERNEL_FLOPS = {"euler_teno": 8250.0}
+# FP64 operations per unit of the compute-bound kernels: what the SQ counters
+# give for a TENO face (profiles/rhs_air5_256_sq_counters.md; FMA-free build).
+# The species sums are formed once per point, the selections without divisions
+KERNEL_FLOPS = {"euler_teno": 4990.0}
 
 
 def parse():

@@ -19,9 +19,9 @@
 //     pair of one column at once.
 // 30 species, 180 reactions, against 64 lanes of the group kernel before:
 // 12^3 cells, FP64, central differences 1033 -> 197 ms; 20^3 cells, FP32 and
-// refinement, analytic Jacobian 576 -> 155 ms; 32^3 cells 5150 -> 2470 ms (FP64,
-// differences), 1435 -> 571 ms (FP64, analytic), 1298 -> 539 ms (refined,
-// analytic).  Still bound by latency: of 220000 cycles of a step with the
+// refinement, analytic Jacobian 576 -> 155 ms; 32^3 cells over 1e-5 s 5153 -> 1686
+// ms (FP64, differences), 1435 -> 374 ms (FP64, analytic), 1298 -> 349 ms (refined,
+// analytic: the refinement's own share of that is 7 %).  Still bound by latency: of 220000 cycles of a step with the
 // analytic Jacobian the factorisation takes 45000, the solves 73000, the
 // Jacobian 40000; with differences the Newtons' chain takes 184000 of 475000.
 #pragma once
@@ -1017,6 +1017,12 @@ struct ChemWave {
 
 // A block per cell in flight: the first wave takes cells from the queue counter
 // until it passes n; with the central-difference Jacobian three more waves help.
+// Waves per SIMD: with differences three, although the registers then spill 300 to
+// 384 B a lane (12^3 cells FP64 274 ms, 20^3 686; two 303 and 814, one 398 and 1276,
+// four 309 and 726): what waits for the Newton chain of one cell is filled by other
+// cells.  With the analytic Jacobian two (36 to 68 B; 20^3 refined 174 ms, 32^3 540;
+// one 221 and 745, three 204 and 613, four 243 and 793): a wave is busy 46 % of its
+// cycles there, and spills cost more than a third wave brings.
 template<class MX, int PREC, bool AJ>
 __global__ void __launch_bounds__(AJ ? 64 : 64*CHEM_FD_WAVES, AJ ? 2 : 3)
 chem_wave_kernel(const htr_fields f, const DMix *__restrict__ mix, const Geo g, double dt, htr_view nsteps,

@@ -307,8 +307,11 @@ struct Diffusion {
 
 // All three directions.  Each face is formed twice, which costs 1400 FP64
 // operations more per cell and saves two thirds of the passes over memory.
-// Bound by the loads' address cycles (16 per 64-lane 8-byte load, 270 loads per
-// cell) and FP64 issue at two waves per SIMD.
+// Bound by the loads' address cycles (16 per 64-lane 8-byte load; a wave issues 481
+// where it straddles a range of the polynomials, counted) and FP64 issue at two
+// waves per SIMD.  With the walks along lines before it in brackets: 256^3 air 3.7
+// (4.8) ms, 4.5 about 6000 K; 512x256x128 boundary layer 3.8 (4.8) ms; 117x93x75
+// air 195 (315) us; 32^3 one species 11 (102) us.
 //
 // The faces of a cell lie between temperatures, so in a flow about a range
 // switch of the polynomials most waves straddle it.  Their coefficients come

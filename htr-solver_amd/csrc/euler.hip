@@ -434,18 +434,18 @@ __device__ inline void store_face(double *__restrict__ F, int64_t nfaces, uint32
 }
 
 // Pass 1 of the hybrid scheme: the hybrid sensor of every face; faces that
-// need TENO are appended to a compacted list.  A block takes 4096 faces and
-// reserves its list range with one atomic (one per wave would serialise some
+// need TENO are appended to a compacted list.  A block takes 256 PT faces (4096)
+// and reserves its list range with one atomic (one per wave would serialise some
 // 10^5 atomics on one address).  The TENO passes gather the six stencil
 // points of every listed face, so the list keeps faces that share stencil
-// rows together: for the y and z sweeps a block's faces are a tile of 64
-// x-cells x 8 faces along the sweep x 8 cells of the remaining direction
-// (a wave takes one x-row of the tile); for the x sweep, whose stencil runs
-// along the row, 4096 consecutive face ids.  A box too small to give every CU
-// a block of that size takes tiles of 1024 or 256 faces, four or one a thread
-// (a block's atomic costs 12 ns in line with the others', a round of dependent
-// loads 1 us): ten blocks of sixteen rounds took 19.8 us for the x faces of a
-// 200^2 box, in tiles of 256 it takes 4.0; 5001-cell tube 16.8 -> 3.5 us.
+// rows together: for the y and z sweeps a block's faces are a tile of TX = 16
+// x-cells x TJ = 2 PT faces along the sweep x 8 cells of the remaining direction
+// (a wave takes four x-rows of the tile); for the x sweep, whose stencil runs
+// along the row, 256 PT consecutive face ids.  A box too small to give every CU
+// a block of 4096 faces takes PT = 4 or 1 in place of 16 (a block's atomic costs 12
+// ns in line with the others', a round of dependent loads 1 us): ten blocks of
+// sixteen rounds took 19.8 us for the x faces of a 200^2 box, in tiles of 256 it
+// takes 4.0; 5001-cell tube 16.8 -> 3.5 us.
 
 template<int DIR, int PT, int TX = 16, int TJ = 2*PT>
 struct ClsTiles {
@@ -544,7 +544,9 @@ euler_classify_kernel(const htr_fields f, const Geo g, int64_t nfaces, int32_t *
 // loads of a component are independent of each other, no thread waits for
 // another, and a small box has a thread per cell instead of one per eight.
 // Bound by the number of loads: a 64-lane 8-byte load takes the CU's address
-// unit 16 cycles (measured, from L1, contiguous or not), 230 of them per cell.
+// unit 16 cycles (measured, from L1, contiguous or not), and a wave of 64 cells
+// issues 335 (counted, 256^3 air), 5400 of the 8700 cycles that a CU has for them;
+// the rest is L2 latency at three waves per SIMD.
 // All three directions, measured with the walks in brackets: 256^3 air 3.9
 // (5.0) ms, 512x256x128 boundary layer 2.9 (4.6) ms, 32^3 one species 15 (155)
 // us; one direction of 256^3 air without TENO faces 1.2 (1.66) ms.

@@ -5,12 +5,14 @@ remarks (one block per kernel: VGPRs, AGPRs, ScratchSize, Occupancy) go to
 _build/resources.log.  check() summarises them and fails when an Euler or
 diffusion kernel uses scratch (register spills or a private array indexed at
 run time): the flux kernels are laid out so that their working set stays in
-registers, and a kernel that spills has regressed.
+registers, and a kernel that spills has regressed.  The implicit chemistry of a
+wave per cell spills by choice (its launch bounds), up to a limit.
 """
 import re
 import sys
 
-NO_SCRATCH = ("euler_", "face_divergence", "diffusion_")
+# bytes a lane
+SCRATCH = {"euler_": 0, "face_divergence": 0, "diffusion_": 0, "chem_wave": 400}
 FIELDS = ("VGPRs", "AGPRs", "ScratchSize [bytes/lane]", "Occupancy [waves/SIMD]")
 
 
@@ -34,10 +36,10 @@ def check(path, verbose=False):
         if verbose:
             print("%-90s vgpr %3d agpr %3d scratch %4d occ %d" % (name[:90], v["VGPRs"], v["AGPRs"],
                   v["ScratchSize [bytes/lane]"], v["Occupancy [waves/SIMD]"]))
-        if any(k in name for k in NO_SCRATCH) and v["ScratchSize [bytes/lane]"] > 0:
+        if any(k in name and v["ScratchSize [bytes/lane]"] > limit for k, limit in SCRATCH.items()):
             bad.append((name, v["ScratchSize [bytes/lane]"]))
     if bad:
-        raise RuntimeError("flux kernels using scratch: " + ", ".join("%s (%d B/lane)" % b for b in bad))
+        raise RuntimeError("kernels using more scratch than their limit: " + ", ".join("%s (%d B/lane)" % b for b in bad))
     return kernels
 
 
