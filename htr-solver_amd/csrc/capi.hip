@@ -1057,7 +1057,7 @@ int htr_workspace_reserve(const htr_grid *g, const htr_fields *f, const htr_mix 
    if ((rc = workspace_faces(*w, fit ? 0 : need.faces_one, need.list, need.teno))) return rc;
    if ((rc = workspace_enthalpy(*w, need.hbuf))) return rc;
    if (g_overlap) {
-      // the side streams of the full RHS, one direction's TENO faces each
+      // the side streams of the full RHS: one direction's list and records each
       RhsAux *aux = rhs_aux((hipStream_t)stream);
       if (!aux) return HTR_E_DEVICE;
       for (int d = 0; d < 3; d++) {
